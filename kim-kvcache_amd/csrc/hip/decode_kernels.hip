@@ -5,10 +5,11 @@
 // KV pages.  Work unit: a workgroup per (lane, chunk of tokens, group of four
 // kv heads); wave w owns kv head h and that head's query group.
 //
-// Fast path (head_dim 64, group <= 16, page-aligned table): per 64-token tile
-//   S^T[token][q] = K[token][:] . Q[q][:]   -> 4 x 2 MFMA 16x16x32 f16
-//   online softmax (base 2) on the 16 scores each lane holds
-//   O^T[d][q]    += V^T[d][token] . P[q][token] -> 2 x 4 x 2 MFMA 16x16x32 f16
+// Fast path (head_dim 64 or 128, group <= 16, page-aligned table): per step
+// of 64 tokens (32 at head_dim 128: the same bytes and operand registers)
+//   S^T[token][q] = K[token][:] . Q[q][:]   -> 8 MFMA 16x16x32 f16
+//   online softmax (base 2) on the 16 (8) scores each lane holds
+//   O^T[d][q]    += V^T[d][token] . P[q][token] -> 16 MFMA 16x16x32 f16
 //                   (P split into fp16 hi and lo parts: ~fp32 weights)
 // K rows and V^T rows (V is stored transposed in the page) are read with
 // 16-byte loads straight into MFMA operand registers; the token order inside
@@ -40,16 +41,20 @@ constexpr unsigned kWholeLaneMax = 1024;   // tokens: longest lane a small batch
 constexpr float kWeightShift = 15.0f;
 
 // ---------------------------------------------------------------------------
-// Fast path for one wave: kv head h, head_dim 64, group <= 16.
+// Fast path for one wave: kv head h, head_dim 64 or 128, group <= 16.
 // ---------------------------------------------------------------------------
 // Online-softmax state of one wave over its tokens: lane (a, r) holds
 // O^T[d][r] for d = 16 db + 4 a + i in acc[db][i], and the running max m and
 // denominator l of query column r (the same in every lane group a).
+template <uint32_t kDim>
 struct WavePartial {
-    float4_t acc[4];
+    float4_t acc[kDim / 16];
     float m;
     float l;
 };
+
+// Head dims with a matrix-core path; the others take the generic path.
+constexpr bool fast_head_dim(uint32_t dim) { return dim == 64 || dim == 128; }
 
 // A K or V^T operand load: non-temporal (streamed past the caches) for long
 // chunks and large launches, where every byte is read once and the
@@ -84,15 +89,40 @@ struct NewTokenRows {
     uint32_t t;
 };
 
+// Eight halves of a caller's row (query, new K row).  The callers' addresses
+// carry no alignment promise; head_dim 64 has always read them as 16-byte
+// vectors, head_dim 128 does so when the address allows it.
+template <uint32_t kDim>
+__device__ inline half8_t load_row8(const uint16_t* p)
+{
+    if (kDim == 64 || (reinterpret_cast<uintptr_t>(p) & 15u) == 0) return load_half8(p);
+    half8_t v;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) v[i] = __builtin_bit_cast(_Float16, p[i]);
+    return v;
+}
+
 // Tokens [c0, c1) of kv head h; the group table starts at token g0 (c0 - g0
 // is a multiple of 64).  When nt.t == c1 - 1 the last token's K and V come
 // from nt's rows (its page group may hold anything at that position).
-template <bool kStream>
-__device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupResolver& res,
-                                       const kimkv_decode_item& item, uint32_t h, uint32_t G, uint32_t g0,
-                                       uint32_t c0, uint32_t c1, NewTokenRows const& nt)
+//
+// Bound by HBM and, for short chunks, by the latency of a step's loads, not
+// by the MFMAs.  kDim = 128 keeps the registers of kDim = 64 by taking 32
+// tokens a step: a step is 16 KiB of K/V per wave either way, two steps in
+// flight.  16 lanes of 500..4000 tokens, 8 kv heads x 128, 4 query heads each
+// (137 MB): 42.5 us with the merge, 1205 us on the generic path, which reads
+// K and V once per query head in 2-byte loads.
+template <uint32_t kDim, bool kStream>
+__device__ WavePartial<kDim> decode_wave_fast(const GroupEntry* groups, const GroupResolver& res,
+                                              const kimkv_decode_item& item, uint32_t h, uint32_t G, uint32_t g0,
+                                              uint32_t c0, uint32_t c1, NewTokenRows const& nt)
 {
-    constexpr uint32_t D = 64;
+    static_assert(kDim == 64 || kDim == 128, "fast path head dims");
+    constexpr uint32_t D = kDim;
+    constexpr uint32_t kKB = 128 / D;        // 32-token blocks per step
+    constexpr uint32_t kStep = 32 * kKB;     // tokens per step
+    constexpr uint32_t kPanels = D / 32;     // K column blocks
+    constexpr uint32_t kDb = D / 16;         // 16-dim blocks of O
     uint32_t const l = threadIdx.x & 63u;
     uint32_t const a = l >> 4;            // lane group
     uint32_t const r = l & 15u;           // row/column inside a 16-wide MFMA tile
@@ -103,19 +133,20 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
     bool const has_new = nt.t != kNoToken && nt.t + 1 == c1;
     uint32_t const new_t = has_new ? nt.t : kNoToken;
 
-    half8_t qb0 = {};
-    half8_t qb1 = {};
+    half8_t qb[kPanels] = {};
     if (qvalid) {
-        qb0 = load_half8(item.query + static_cast<uint64_t>(q) * D + a * 8);
-        qb1 = load_half8(item.query + static_cast<uint64_t>(q) * D + 32 + a * 8);
+#pragma unroll
+        for (uint32_t j = 0; j < kPanels; ++j) {
+            qb[j] = load_row8<D>(item.query + static_cast<uint64_t>(q) * D + 32 * j + a * 8);
+        }
     }
     float const scale2 = item.attention_scale * kLog2e;
     float m_run = -INFINITY;
     float l_part = 0.0f;
-    float4_t acc[4] = {};
+    float4_t acc[kDb] = {};
     half8_t const zero8 = {};
 
-    // One 64-token step is a load phase (K rows and V^T rows of the step into
+    // One step is a load phase (K rows and V^T rows of the step into
     // registers) and a compute phase; the next step's loads are issued before
     // the current step's compute (two register buffers), so each wave keeps
     // up to two steps of K/V in flight and the compute hides under them.  The
@@ -124,32 +155,34 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
     // group of the chunk is mapped), so the waits before a compute cover
     // exactly the older buffer's loads.
     struct Ops {
-        half8_t k[2][2][2];
-        half8_t v[2][4];
+        half8_t k[kKB][2][kPanels];
+        half8_t v[kKB][kDb];
     };
     auto load = [&](Ops& o, uint32_t t0, auto tail) {
         constexpr bool kTail = decltype(tail)::value;
         uint32_t const tg = (t0 - g0) >> 3;
         uint32_t const nvalid = c1 - t0;
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < kKB; ++kb) {
             GroupEntry const gk = groups[tg + 4 * kb + x];
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
                 uint32_t const tt = 32 * kb + 8 * x + 4 * e + (l & 3u);
                 if (kTail && t0 + tt == new_t) {
-                    // The new token's K row: dims [8a, 8a+8) and [32+8a, 40+8a) of the source.
-                    o.k[kb][e][0] = load_half8(nt.key + a * 8);
-                    o.k[kb][e][1] = load_half8(nt.key + 32 + a * 8);
+                    // The new token's K row: dims [32j+8a, 32j+8a+8) of the source.
+#pragma unroll
+                    for (uint32_t j = 0; j < kPanels; ++j) o.k[kb][e][j] = load_row8<D>(nt.key + 32 * j + a * 8);
                 } else if (!kTail || (tt < nvalid && gk.page != kUnmappedGroup)) {
-                    // K column blocks of 32 dims: dims [8a, 8a+8) and [32+8a, 40+8a).
+                    // K column blocks of 32 dims: dims [32j+8a, 32j+8a+8).
                     const uint16_t* row = res.block(gk) + static_cast<uint64_t>(gk.pt0 + 4 * e + (l & 3u)) * 32
                         + a * 8;
-                    o.k[kb][e][0] = load_kv<kStream>(row);
-                    o.k[kb][e][1] = load_kv<kStream>(row + static_cast<uint64_t>(gk.cap) * 32);
+#pragma unroll
+                    for (uint32_t j = 0; j < kPanels; ++j) {
+                        o.k[kb][e][j] = load_kv<kStream>(row + static_cast<uint64_t>(gk.cap) * (32 * j));
+                    }
                 } else {
-                    o.k[kb][e][0] = zero8;
-                    o.k[kb][e][1] = zero8;
+#pragma unroll
+                    for (uint32_t j = 0; j < kPanels; ++j) o.k[kb][e][j] = zero8;
                 }
             }
             GroupEntry const gv = groups[tg + 4 * kb + a];
@@ -159,12 +192,12 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
                 uint32_t const vw = v_width(gv.cap);
                 const uint16_t* vt = res.block(gv) + v_offset(gv.cap, D, gv.pt0, r);
 #pragma unroll
-                for (uint32_t db = 0; db < 4; ++db) {
+                for (uint32_t db = 0; db < kDb; ++db) {
                     o.v[kb][db] = load_kv<kStream>(vt + static_cast<uint64_t>(db * 16) * vw);
                 }
             } else {
 #pragma unroll
-                for (uint32_t db = 0; db < 4; ++db) o.v[kb][db] = zero8;
+                for (uint32_t db = 0; db < kDb; ++db) o.v[kb][db] = zero8;
             }
         }
     };
@@ -174,12 +207,12 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
         if (kTail) {
             // Tokens past the chunk end may hold stale data: zero their V.
 #pragma unroll
-            for (uint32_t kb = 0; kb < 2; ++kb) {
+            for (uint32_t kb = 0; kb < kKB; ++kb) {
                 uint32_t const vt0 = 32 * kb + 8 * a;
                 if (vt0 < nvalid && vt0 + 8 > nvalid) {
                     uint32_t const keep = nvalid - vt0;
 #pragma unroll
-                    for (uint32_t db = 0; db < 4; ++db) {
+                    for (uint32_t db = 0; db < kDb; ++db) {
 #pragma unroll
                         for (uint32_t j = 0; j < 8; ++j) {
                             if (j >= keep) o.v[kb][db][j] = static_cast<_Float16>(0.0f);
@@ -190,19 +223,22 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
         }
 
         // ---- scores ----
-        float4_t s[2][2];
+        float4_t s[kKB][2];
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
                 float4_t z = {};
-                z = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.k[kb][e][0], qb0, z, 0, 0, 0);
-                s[kb][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.k[kb][e][1], qb1, z, 0, 0, 0);
+#pragma unroll
+                for (uint32_t j = 0; j < kPanels; ++j) {
+                    z = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.k[kb][e][j], qb[j], z, 0, 0, 0);
+                }
+                s[kb][e] = z;
             }
         }
         float mx = -INFINITY;
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
 #pragma unroll
@@ -217,7 +253,10 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         float const m_new = fmaxf(m_run, mx);
-        float const alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        // Head dim 128, as the generic path: while every score is -inf the
+        // reference is 0, so the weights are zeros and not NaN.
+        float const m_top = kDim == 128 && m_new == -INFINITY ? 0.0f : m_new;
+        float const alpha = __builtin_amdgcn_exp2f(m_run - m_top);
         m_run = m_new;
 
         // Weights p = 2^(s - m + kWeightShift) <= 2^15 go to the MFMA as two
@@ -225,12 +264,12 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
         // products with V carry ~22 significant bits, like the fp32 weights
         // of the reference, and the denominator sums the same p.  The shift
         // keeps small weights in fp16's normal range; it cancels in o / l.
-        float const m_ref = m_new - kWeightShift;
-        half8_t pb[2];
-        half8_t pl[2];
+        float const m_ref = m_top - kWeightShift;
+        half8_t pb[kKB];
+        half8_t pl[kKB];
         float psum = 0.0f;
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
 #pragma unroll
@@ -245,13 +284,13 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
         }
         l_part = l_part * alpha + psum;
 #pragma unroll
-        for (uint32_t db = 0; db < 4; ++db) acc[db] *= alpha;
+        for (uint32_t db = 0; db < kDb; ++db) acc[db] *= alpha;
 
         // ---- O^T += V^T . (P_hi + P_lo)^T ----
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < kKB; ++kb) {
 #pragma unroll
-            for (uint32_t db = 0; db < 4; ++db) {
+            for (uint32_t db = 0; db < kDb; ++db) {
                 acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.v[kb][db], pb[kb], acc[db], 0, 0, 0);
                 acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.v[kb][db], pl[kb], acc[db], 0, 0, 0);
             }
@@ -260,39 +299,39 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
     Ops buf_a;
     Ops buf_b;
     std::false_type const full{};
-    uint32_t const nfull = (has_new ? c1 - c0 - 1 : c1 - c0) >> 6;
+    uint32_t const nfull = (has_new ? c1 - c0 - 1 : c1 - c0) / kStep;
     if (nfull > 0) {
         // At the top of each round buf_a holds step s - 1 in flight; the body
         // has no bounds test, so no load in it is conditional.
         load(buf_a, c0, full);
         uint32_t s = 1;
         for (; s + 1 < nfull; s += 2) {
-            load(buf_b, c0 + 64 * s, full);
+            load(buf_b, c0 + kStep * s, full);
             compute(buf_a, c0, full);
-            load(buf_a, c0 + 64 * (s + 1), full);
+            load(buf_a, c0 + kStep * (s + 1), full);
             compute(buf_b, c0, full);
         }
         if (s < nfull) {
-            load(buf_b, c0 + 64 * s, full);
+            load(buf_b, c0 + kStep * s, full);
             compute(buf_a, c0, full);
             compute(buf_b, c0, full);
         } else {
             compute(buf_a, c0, full);
         }
     }
-    if (c0 + 64 * nfull < c1) {
-        uint32_t const t0 = c0 + 64 * nfull;
+    if (c0 + kStep * nfull < c1) {
+        uint32_t const t0 = c0 + kStep * nfull;
         load(buf_a, t0, std::true_type{});
         if (has_new) {
             // V^T rows d = 16 db + r of the new token's 8-token group: element
             // j of lane group a (tokens [32 kb + 8 a, +8) of the step) is the
             // new token for one (kb, a).
 #pragma unroll
-            for (uint32_t kb = 0; kb < 2; ++kb) {
+            for (uint32_t kb = 0; kb < kKB; ++kb) {
                 uint32_t const j = new_t - t0 - (32 * kb + 8 * a);
                 if (j < 8) {
 #pragma unroll
-                    for (uint32_t db = 0; db < 4; ++db) {
+                    for (uint32_t db = 0; db < kDb; ++db) {
                         buf_a.v[kb][db][j] = __builtin_bit_cast(_Float16, nt.value[16 * db + r]);
                     }
                 }
@@ -303,9 +342,9 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
 
     float l_tot = l_part + __shfl_xor(l_part, 16);
     l_tot += __shfl_xor(l_tot, 32);
-    WavePartial out;
+    WavePartial<D> out;
 #pragma unroll
-    for (uint32_t db = 0; db < 4; ++db) out.acc[db] = acc[db];
+    for (uint32_t db = 0; db < kDb; ++db) out.acc[db] = acc[db];
     out.m = m_run;
     out.l = l_tot;
     return out;
@@ -314,12 +353,13 @@ __device__ WavePartial decode_wave_d64(const GroupEntry* groups, const GroupReso
 // Writes dims [d0, d0 + 4) of query head q: the fp16 output when the lane
 // has one chunk, else the chunk's (o, m, l) partial for combine_kernel (m and
 // l by the one caller per row that passes write_ml).
+template <uint32_t kDim>
 __device__ inline void store_partial(const kimkv_decode_item& item, uint32_t QH, uint32_t q, uint32_t chunk_index,
                                      bool single_chunk, float4_t o, uint32_t d0, float m, float l, bool write_ml)
 {
-    constexpr uint32_t D = 64;
+    constexpr uint32_t D = kDim;
     if (single_chunk) {
-        float const inv = 1.0f / l;
+        float const inv = kDim == 128 && !(l > 0.0f) ? 0.0f : 1.0f / l;   // l = 0 as the generic path
         uint16_t* out = item.output + static_cast<uint64_t>(q) * D + d0;
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) out[i] = __half_as_ushort(__float2half_rn(o[i] * inv));
@@ -556,7 +596,7 @@ struct DecodeLds {
 };
 
 // Builds the group table of tokens [c0, c1) of `item` (c0 a multiple of 8)
-// and returns whether the fast path applies (head_dim 64, group <= 16, every
+// and returns whether the fast path applies (head_dim kDim, group <= 16, every
 // 8-token group mapped and aligned).  With an active write job, groups of
 // its destination page below the copied count are read from the
 // copy-on-write source page instead, and lds.new_ok says whether the chunk's
@@ -565,6 +605,7 @@ struct DecodeLds {
 // position of the new token read as another token, a group mixing copied
 // and kept positions) goes to the generic path, which applies the same rule
 // per token.  Called by every thread of the block.
+template <uint32_t kDim>
 __device__ bool build_chunk_table(const PoolView& P, const kimkv_decode_item& item, uint32_t QH, uint32_t c0,
                                   uint32_t c1, DecodeLds& lds, JobView const& jv)
 {
@@ -636,7 +677,7 @@ __device__ bool build_chunk_table(const PoolView& P, const kimkv_decode_item& it
     if (generic) lds.generic = 1;
     __syncthreads();
     uint32_t const G = QH / P.heads;
-    return P.dim == 64 && G <= 16 && lds.generic == 0;
+    return P.dim == kDim && G <= 16 && lds.generic == 0;
 }
 
 // A kRecords launch's cache of chunk group tables (optional): the table a
@@ -682,12 +723,13 @@ __host__ __device__ inline uint64_t table_cache_chunk_bytes(uint32_t stride)
 // is built from the descriptors, and the chunk's first workgroup (blockIdx.y
 // 0) stores it with the launch's tag and id.  Called by every thread of the
 // block.
+template <uint32_t kDim>
 __device__ inline bool chunk_table_cached(const PoolView& P, const kimkv_decode_item& item, uint32_t QH, uint32_t c0,
                                           uint32_t c1, DecodeLds& lds, JobView const& jv, TableCache const& cache,
                                           uint32_t chunk_id, TableCacheHeader const& s_hdr)
 {
     uint32_t const ngroups = (c1 - c0 + 7) / 8;
-    if (cache.base == nullptr || ngroups > cache.stride) return build_chunk_table(P, item, QH, c0, c1, lds, jv);
+    if (cache.base == nullptr || ngroups > cache.stride) return build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv);
     __syncthreads();   // the header and entries copied into LDS
     uint32_t const G = QH / P.heads;
     if (s_hdr.tag == cache.tag && s_hdr.launch != cache.launch && s_hdr.ngroups == ngroups) {
@@ -696,10 +738,10 @@ __device__ inline bool chunk_table_cached(const PoolView& P, const kimkv_decode_
             lds.new_ok = (s_hdr.flags >> 1) & 1u;
         }
         __syncthreads();
-        return P.dim == 64 && G <= 16 && lds.generic == 0;
+        return P.dim == kDim && G <= 16 && lds.generic == 0;
     }
     __syncthreads();   // every thread has read the header before the table is rebuilt
-    bool const fast = build_chunk_table(P, item, QH, c0, c1, lds, jv);
+    bool const fast = build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv);
     if (blockIdx.y == 0) {
         unsigned char* c = cache.base + table_cache_chunk_bytes(cache.stride) * chunk_id;
         for (uint32_t g = threadIdx.x; g < ngroups; g += kBlock) {
@@ -728,7 +770,7 @@ __device__ inline NewTokenRows new_token_rows(const DecodeLds& lds, JobView cons
     return NewTokenRows{jv.key + static_cast<uint64_t>(h) * D, jv.value + static_cast<uint64_t>(h) * D, T - 1};
 }
 
-template <bool kStream>
+template <uint32_t kDim, bool kStream>
 __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t QH,
                                         uint32_t c0, uint32_t c1, uint32_t chunk_index, bool single, bool fast,
                                         DecodeLds& lds, JobView const& jv)
@@ -745,52 +787,56 @@ __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_it
     uint32_t const quarter = ((c1 - c0 + 3) / 4 + 63) / 64 * 64;
     uint32_t const s0 = min(c0 + wave * quarter, c1);
     uint32_t const s1 = min(s0 + quarter, c1);
-    WavePartial w;
+    WavePartial<kDim> w;
     if (s0 < s1) {
-        w = decode_wave_d64<kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, s0, s1,
-                                     new_token_rows(lds, jv, item.token_count, h, 64));
+        w = decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, s0, s1,
+                                            new_token_rows(lds, jv, item.token_count, h, kDim));
     } else {
 #pragma unroll
-        for (uint32_t db = 0; db < 4; ++db) w.acc[db] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t db = 0; db < kDim / 16; ++db) w.acc[db] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         w.m = -INFINITY;
         w.l = 0.0f;
     }
     // Every wave is done with the group table: its LDS holds the four states,
-    // [wave][query column][68 floats: o(64), m, l, pad].
-    constexpr uint32_t kRow = 68;
+    // [wave][query column][kDim + 4 floats: o(kDim), m, l, pad].
+    constexpr uint32_t kRow = kDim + 4;
+    static_assert(4 * 16 * kRow * sizeof(float) <= sizeof(lds.groups), "the states fit the group table's space");
     __syncthreads();
     float* part = reinterpret_cast<float*>(lds.groups);
     {
         uint32_t const l = tid & 63u;
         float* row = part + (wave * 16 + (l & 15u)) * kRow;
 #pragma unroll
-        for (uint32_t db = 0; db < 4; ++db) {
+        for (uint32_t db = 0; db < kDim / 16; ++db) {
             *reinterpret_cast<float4_t*>(row + db * 16 + 4 * (l >> 4)) = w.acc[db];
         }
         if (l < 16) {
-            row[64] = w.m;
-            row[65] = w.l;
+            row[kDim] = w.m;
+            row[kDim + 1] = w.l;
         }
     }
     __syncthreads();
-    // Thread t merges dims [4 (t % 16), +4) of query column t / 16.
+    // Thread t merges dims [4 (t % 16) + 64 j, +4) of query column t / 16.
     uint32_t const r = tid >> 4;
-    uint32_t const d0 = (tid & 15u) * 4;
     if (r >= G) return;
     float M = -INFINITY;
 #pragma unroll
-    for (uint32_t v = 0; v < kHeadsPerBlock; ++v) M = fmaxf(M, part[(v * 16 + r) * kRow + 64]);
-    float den = 0.0f;
-    float4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t v = 0; v < kHeadsPerBlock; ++v) M = fmaxf(M, part[(v * 16 + r) * kRow + kDim]);
 #pragma unroll
-    for (uint32_t v = 0; v < kHeadsPerBlock; ++v) {
-        const float* row = part + (v * 16 + r) * kRow;
-        float const m = row[64];
-        float const c = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
-        den += c * row[65];
-        o += c * *reinterpret_cast<const float4_t*>(row + d0);
+    for (uint32_t j = 0; j < kDim / 64; ++j) {
+        uint32_t const d0 = (tid & 15u) * 4 + 64 * j;
+        float den = 0.0f;
+        float4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (uint32_t v = 0; v < kHeadsPerBlock; ++v) {
+            const float* row = part + (v * 16 + r) * kRow;
+            float const m = row[kDim];
+            float const c = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+            den += c * row[kDim + 1];
+            o += c * *reinterpret_cast<const float4_t*>(row + d0);
+        }
+        store_partial<kDim>(item, QH, h * G + r, chunk_index, single, o, d0, M, den, d0 == 0);
     }
-    store_partial(item, QH, h * G + r, chunk_index, single, o, d0, M, den, d0 == 0);
 }
 
 // Stores the lane's new token for kv heads [h0, h1) of `layer` (a job that
@@ -862,6 +908,8 @@ static_assert(sizeof(DecodeLaneSlot) == KIMKV_DECODE_LANE_SLOT_BYTES, "slot size
 // none): every chunk reads the positions the job writes from the job's
 // sources, and the workgroups of the chunk that holds the lane's last token
 // store them after their reads.
+// kDim: the head dim of the fast path (64 or 128); a storage of another head
+// dim runs the kDim = 64 instance, whose workgroups all take the generic path.
 // kStream: non-temporal K/V loads (load_kv).
 // slots: when non-null, each lane's merge record (DecodeLaneSlot, tagged
 // `tag`) for the merge launch.
@@ -936,7 +984,7 @@ __device__ inline void record_lane(const kimkv_decode_lane& r, const kimkv_decod
     }
 }
 
-template <bool kSplit, bool kStream, LaneSource kSrc>
+template <uint32_t kDim, bool kSplit, bool kStream, LaneSource kSrc>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_kernel(
     PoolView P, const kimkv_decode_item* items, const uint32_t* prefix, uint32_t lane_count, uint32_t chunk_tokens,
     uint32_t QH, float* partials, const kimkv_append_job* writes, DecodeLaneSlot* slots, uint64_t tag,
@@ -1090,9 +1138,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     if (tid == 0) lds.job = job;   // visible after build_chunk_table's barriers
     bool fast;
     if constexpr (kSrc == LaneSource::kRecords) {
-        fast = chunk_table_cached(P, item, QH, c0, c1, lds, jv, sa.cache, chunk_id, s_cache_hdr);
+        fast = chunk_table_cached<kDim>(P, item, QH, c0, c1, lds, jv, sa.cache, chunk_id, s_cache_hdr);
     } else {
-        fast = build_chunk_table(P, item, QH, c0, c1, lds, jv);
+        fast = build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv);
     }
 
     uint32_t const wave = tid >> 6;
@@ -1101,20 +1149,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         if (h < H && !fast) {
             decode_wave_generic(P, item, h, G, QH, c0, c1, chunk_index, single, &lds.wave_tokens[wave], jv);
         } else if (h < H) {
-            WavePartial const w = decode_wave_d64<kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G,
-                                                           c0, c0, c1, new_token_rows(lds, jv, T, h, 64));
+            WavePartial<kDim> const w =
+                decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, c0, c1,
+                                                new_token_rows(lds, jv, T, h, kDim));
             uint32_t const l = tid & 63u;
             uint32_t const r = l & 15u;
             if (r < G) {
 #pragma unroll
-                for (uint32_t db = 0; db < 4; ++db) {
-                    store_partial(item, QH, h * G + r, chunk_index, single, w.acc[db], db * 16 + 4 * (l >> 4), w.m,
-                                  w.l, db == 0 && l < 16);
+                for (uint32_t db = 0; db < kDim / 16; ++db) {
+                    store_partial<kDim>(item, QH, h * G + r, chunk_index, single, w.acc[db], db * 16 + 4 * (l >> 4),
+                                        w.m, w.l, db == 0 && l < 16);
                 }
             }
         }
     } else if (blockIdx.y < H) {
-        decode_head_split_chunk<kStream>(P, item, blockIdx.y, QH, c0, c1, chunk_index, single, fast, lds, jv);
+        decode_head_split_chunk<kDim, kStream>(P, item, blockIdx.y, QH, c0, c1, chunk_index, single, fast, lds, jv);
     }
     // The job comes back from LDS rather than staying in registers across
     // the streaming loop.
@@ -1148,6 +1197,7 @@ __host__ __device__ inline uint32_t guided_edge(uint32_t T, uint32_t n, uint32_t
 // unit is a head-split chunk whose partial goes to the lane's slot k; the
 // merge launch combines the slices.  The last workgroup to leave resets the
 // counter slot for the next launch that uses it.
+template <uint32_t kDim>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_guided_kernel(
     PoolView P, const kimkv_decode_item* items, const uint32_t* prefix, uint32_t lane_count, uint32_t total_chunks,
     uint32_t QH, float* partials, uint32_t* counter, const kimkv_append_job* writes)
@@ -1192,17 +1242,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         JobView const jv = job_view(P, job, job_ok);
         if (tid == 0) lds.job = job;   // the previous unit ended with a barrier
         if (c0 >= c1) {
-            // An empty slice still leaves its partial: weight zero in the merge.
-            uint32_t const r = tid >> 4;
-            uint32_t const d0 = (tid & 15u) * 4;
-            if (r < G) {
-                store_partial(item, QH, h * G + r, k, false, float4_t{0.0f, 0.0f, 0.0f, 0.0f}, d0, -INFINITY, 0.0f,
-                              d0 == 0);
-            }
+            // An empty slice still leaves its partial, for any head dim and
+            // group: weight zero in the merge.
+            float* ws = item.workspace + (static_cast<uint64_t>(k) * QH + static_cast<uint64_t>(h) * G) * (D + 2);
+            for (uint32_t i = tid; i < G * (D + 2); i += kBlock) ws[i] = i % (D + 2) == D ? -INFINITY : 0.0f;
             continue;
         }
-        bool const fast = build_chunk_table(P, item, QH, c0, c1, lds, jv);
-        decode_head_split_chunk<true>(P, item, h, QH, c0, c1, k, n == 1, fast, lds, jv);
+        bool const fast = build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv);
+        decode_head_split_chunk<kDim, true>(P, item, h, QH, c0, c1, k, n == 1, fast, lds, jv);
         // The last slice (never empty) stores the job's positions of head h.
         if (writer && job_ok) write_token_heads(P, lds.job, item.layer, h, h + 1);
         __syncthreads();   // the next unit rebuilds the table in the same LDS
@@ -1457,6 +1504,7 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
     if (total_chunks == 0) return KIMKV_OK;
     hipStream_t const s = native(stream);
     uint32_t const H = storage->layout.kv_heads;
+    bool const wide = storage->layout.head_dim == 128;   // the kDim = 128 instances; every other dim runs kDim = 64's
     uint64_t const units = static_cast<uint64_t>(lane_count) * H * KIMKV_DECODE_GUIDED_SLICES;
     if (guided && (units > 0x7FFFFFFFu || storage->work_counters == nullptr)) return KIMKV_INVALID_ARGUMENT;
     dim3 const grid(total_chunks, head_split ? H : (H + kHeadsPerBlock - 1) / kHeadsPerBlock);
@@ -1474,9 +1522,16 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
         uint32_t* counter = storage->work_counters + static_cast<size_t>(slot) * kWorkCounterStride;
         uint64_t const resident = 2ull * (storage->compute_units > 0 ? storage->compute_units : 256);
         auto const workers = static_cast<uint32_t>(units < resident ? units : resident);
-        decode_guided_kernel<<<workers, kBlock, 0, s>>>(pool_view(*storage), device_items, device_chunk_prefix,
-                                                         lane_count, total_chunks, query_heads, partials, counter,
-                                                         writes);
+        auto guide = [&](auto dim) {
+            decode_guided_kernel<decltype(dim)::value><<<workers, kBlock, 0, s>>>(
+                pool_view(*storage), device_items, device_chunk_prefix, lane_count, total_chunks, query_heads, partials,
+                counter, writes);
+        };
+        if (wide) {
+            guide(std::integral_constant<uint32_t, 128>{});
+        } else {
+            guide(std::integral_constant<uint32_t, 64>{});
+        }
     } else {
         // Streamed K/V loads for long chunks (a workgroup streams at least
         // 2048 tokens) or more than one round of resident workgroups (two
@@ -1484,7 +1539,8 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
         uint64_t const resident = 2ull * (storage->compute_units > 0 ? storage->compute_units : 256);
         bool const stream_loads = chunk_tokens >= 2048 || static_cast<uint64_t>(grid.x) * grid.y > resident;
         PoolView const pv = pool_view(*storage);
-        auto go = [&](auto split, auto stream_kv, auto src) {
+        auto go = [&](auto dim, auto split, auto stream_kv, auto src) {
+            constexpr uint32_t kD = decltype(dim)::value;
             constexpr bool kS = decltype(split)::value;
             constexpr bool kT = decltype(stream_kv)::value;
             constexpr LaneSource kL = decltype(src)::value;
@@ -1495,17 +1551,24 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
                 sa.layer = *layer_args;
                 sa.cache = cache;
             }
-            decode_kernel<kS, kT, kL><<<grid, kBlock, 0, s>>>(pv, device_items, device_chunk_prefix, lane_count,
-                                                              chunk_tokens, query_heads, partials, writes, slots, tag,
-                                                              lanes, sa);
+            decode_kernel<kD, kS, kT, kL><<<grid, kBlock, 0, s>>>(pv, device_items, device_chunk_prefix, lane_count,
+                                                                  chunk_tokens, query_heads, partials, writes, slots,
+                                                                  tag, lanes, sa);
         };
         auto pick = [&](auto src) {
             using T_ = std::true_type;
             using F_ = std::false_type;
-            if (head_split && stream_loads) go(T_{}, T_{}, src);
-            else if (head_split) go(T_{}, F_{}, src);
-            else if (stream_loads) go(F_{}, T_{}, src);
-            else go(F_{}, F_{}, src);
+            auto modes = [&](auto dim) {
+                if (head_split && stream_loads) go(dim, T_{}, T_{}, src);
+                else if (head_split) go(dim, T_{}, F_{}, src);
+                else if (stream_loads) go(dim, F_{}, T_{}, src);
+                else go(dim, F_{}, F_{}, src);
+            };
+            if (wide) {
+                modes(std::integral_constant<uint32_t, 128>{});
+            } else {
+                modes(std::integral_constant<uint32_t, 64>{});
+            }
         };
         if (records) {
             pick(std::integral_constant<LaneSource, LaneSource::kRecords>{});
@@ -1621,7 +1684,7 @@ kimkv_status kimkv_decode_plan(const kimkv_storage* storage, const uint32_t* tok
     // When four kv heads per workgroup would need split-K but one kv head per
     // workgroup would not, take one head per workgroup with its chunk split
     // over the four waves: same workgroup count, no partials, no merge launch.
-    bool const fast_shape = storage->layout.head_dim == 64 && query_heads % H == 0 && query_heads / H <= 16;
+    bool const fast_shape = fast_head_dim(storage->layout.head_dim) && query_heads % H == 0 && query_heads / H <= 16;
     // The guided persistent mode (KIMKV_DECODE_GUIDED) is not chosen here: at
     // 128 lanes x 32k tokens it measured 0.638 ms per launch (six slices) and
     // 0.652 ms (three) against 0.628 ms for one head-split chunk per lane on

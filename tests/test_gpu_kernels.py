@@ -430,8 +430,8 @@ def test_decode_lane_records_match_item_launch(dev, mode, order, heads, dim):
     strides).  With a chunk table cache: the first launch of a tag builds and stores the tables, the next
     two read them, and a new tag over the same cache rebuilds them; every launch gives the same outputs.
     Malformed launches are refused without running.  With 8 kv heads a chunk has two workgroups of four
-    heads each (or eight in the head-split mode) sharing its cached table; head_dim 128 takes the generic
-    path (and the merge of two dims per lane)."""
+    heads each (or eight in the head-split mode) sharing its cached table; head_dim 128 takes the
+    merge of two dims per lane."""
     shape = (3, heads, dim)
     L, H, D = shape
     QH, layer = 32, 1
@@ -941,6 +941,38 @@ def test_decode_generic_head_dim(dev):
     _decode_case(dev, (1, 2, 128), [90, 1500], G=4, seed=10)
 
 
+@pytest.mark.parametrize("G", [1, 4, 16])
+@pytest.mark.parametrize("mode", ["four_heads", "head_split", "plan"])
+def test_decode_head_dim_128(dev, mode, G):
+    # The 128-dim fast path around its 32-token steps (one, two and several, with and without a tail), the
+    # 64-token quarters of the head-split mode, split-K lanes, five kv heads (a partly empty head block).
+    chunk = {"four_heads": 256, "head_split": 256 | dev.DECODE_HEAD_SPLIT, "plan": None}[mode]
+    _decode_case(dev, (2, 5, 128), [1, 7, 31, 32, 33, 64, 65, 95, 96, 128, 257, 700, 2049], G=G, seed=81, chunk=chunk)
+
+
+def test_decode_head_dim_128_guided(dev):
+    _decode_case(dev, (2, 4, 128), [1, 63, 300, 1000, 5000], G=4, seed=82, chunk=dev.DECODE_GUIDED | 64)
+
+
+@pytest.mark.parametrize("mode", ["four_heads", "head_split"])
+def test_decode_head_dim_128_writes(dev, mode):
+    """The 128-dim fast path's fused token write: outputs and pages as append-then-decode gives them."""
+    shape, G = (2, 4, 128), 4
+    L, H, D = shape
+    T = [5, 8, 31, 32, 63, 64, 100, 700, 1303]
+    alloc = helpers.SlotAllocator(sum(t // 8 + 4 for t in T) + 16 - len(T) - 4, sum(t // 64 + 1 for t in T) + 2,
+                                  seed=83)
+    tables = [helpers.hetero_table(t, alloc) for t in T]
+    news = oracle.synth_rows(len(T) * 2 * H * D, 84, 0, D).reshape(len(T), 2, H, D)
+    layers = [i % L for i in range(len(T))]
+    chunk = {"four_heads": 256, "head_split": 256 | dev.DECODE_HEAD_SPLIT}[mode]
+    a, pa, total = _write_then_decode(dev, False, tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8})
+    b, pb, _ = _write_then_decode(dev, "slots_prefix", tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8})
+    assert total > len(T)
+    for i in range(len(T)):
+        assert np.array_equal(pa[i], pb[i]) and np.array_equal(a[i], b[i]), (mode, i)
+
+
 def test_decode_unaligned_pages_generic(dev):
     # 6-token pages: tables not 8-aligned take the generic path.
     _decode_case(dev, (2, 4, 64), [17, 200, 3000], G=8, micro_tokens=6, extent_tokens=48, seed=12,
@@ -1196,8 +1228,18 @@ def test_prefill_sharp_softmax_stays_in_tolerance(dev):
         _prefill_case(dev, (2, 4, 64), [(300, 64), (1000, 200), (0, 48)], G=8, seed=seed, q_gain=gain)
 
 
+@pytest.mark.parametrize("G", [1, 4, 16])
+def test_prefill_head_dim_128(dev, G):
+    """The 128-dim MFMA path around its 32-key tiles and its blocks of 128 / G tokens, across a group-table
+    segment (4096 keys), and with sharp softmaxes."""
+    _prefill_case(dev, (2, 2, 128), [(0, 1), (0, 32), (31, 33), (100, 65), (7, 129), (64, 16)], G=G, seed=86)
+    _prefill_case(dev, (1, 2, 128), [(4080, 40)], G=G, seed=87)
+    _prefill_case(dev, (1, 2, 128), [(300, 20), (0, 48)], G=G, seed=88, q_gain=6.0)
+
+
 def test_prefill_generic_paths(dev):
-    _prefill_case(dev, (2, 2, 128), [(90, 20)], G=2, seed=26)                 # D != 64
+    _prefill_case(dev, (2, 2, 128), [(90, 20)], G=2, seed=26)                 # D = 128
+    _prefill_case(dev, (2, 2, 96), [(90, 20)], G=2, seed=26)                  # D != 64, 128
     _prefill_case(dev, (2, 1, 64), [(50, 9)], G=3, seed=27)                   # G does not divide 16
     _prefill_case(dev, (2, 4, 64), [(17, 30)], G=8, micro_tokens=6, extent_tokens=48, seed=28,
                   uniform_pages=True)                                          # unaligned pages
