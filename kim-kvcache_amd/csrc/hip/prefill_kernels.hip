@@ -22,8 +22,14 @@
 // per column (only on the diagonal tiles).  The group table (8-token groups
 // of the key range, resolved to K and V^T pointers of the block's head) is
 // built in LDS one 4096-key segment at a time.
+// Head dim 128 walks 32-key tiles (the same 16 KiB, the same staging
+// registers) and hands its softmax weights to the matrix cores in two fp16
+// parts, so that they keep the precision of fp32 weights (two ragged chunks
+// of up to 256 tokens on contexts of up to 1500, 8 kv heads x 128, 4 query
+// heads each: 35.8 us, 4440 us on the generic path).
 // Tables that do not keep 8-token groups aligned, head dims other than 64 and
-// group sizes that do not divide 16 take a one-row-at-a-time generic path.
+// 128 and group sizes that do not divide 16 take a one-row-at-a-time generic
+// path.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,19 +46,33 @@ namespace {
 constexpr unsigned kBlock = 256;   // 4 waves
 constexpr unsigned kWaves = kBlock / 64;
 constexpr unsigned kColBlocks = 2;  // 16-column MFMA blocks per wave
-constexpr unsigned kTileKeys = 64;
 constexpr float kLazyRescaleLog2 = 8.0f;
+
+// What depends on the head dim of the MFMA path (64 or 128).
+template <uint32_t kDim>
+struct PrefillDims {
+    static_assert(kDim == 64 || kDim == 128, "MFMA path head dims");
+    static constexpr uint32_t kTileKeys = 4096 / kDim;   // keys per staged tile: 16 KiB of K and V^T
+    static constexpr uint32_t kKB = kTileKeys / 32;      // 32-key halves of a tile
+    static constexpr uint32_t kPanels = kDim / 32;       // 32-dim column blocks of K
+    static constexpr uint32_t kDb = kDim / 16;           // 16-dim blocks of O
+    // Softmax weights as two fp16 parts, p = hi + lo (~22 bits, where the
+    // generic path these shapes took before holds fp32 weights); the weights
+    // are then shifted up so that lo stays a normal number for small ones.
+    static constexpr bool kSplitP = kDim == 128;
+    static constexpr float kWeightShift = kSplitP ? 7.0f : 0.0f;
+};
 
 struct PrefillShape {
     uint32_t tpw;        // new tokens per 16-column block
     uint32_t G;          // query heads per KV head
-    bool mfma;           // D == 64 and G divides 16
+    bool mfma;           // D is 64 or 128 and G divides 16
 };
 
 __host__ __device__ inline PrefillShape prefill_shape(uint32_t QH, uint32_t H, uint32_t D)
 {
     uint32_t const G = QH / H;
-    bool const mfma = D == 64 && G >= 1 && G <= 16 && 16 % G == 0;
+    bool const mfma = (D == 64 || D == 128) && G >= 1 && G <= 16 && 16 % G == 0;
     return PrefillShape{mfma ? 16 / G : 1, G, mfma};
 }
 
@@ -61,28 +81,38 @@ __host__ __device__ inline uint32_t prefill_block_tokens(PrefillShape s)
     return s.mfma ? kWaves * kColBlocks * s.tpw : kWaves;
 }
 
-// One 64-key tile of one KV head (D = 64) staged in LDS, in 16-byte units:
-//   K   unit (key t, dim octet o) at t * 8 + (o ^ k_swizzle(t))
-//   V^T unit (dim d, key octet c) at d * 8 + (c ^ (d & 7))
+// One tile of one KV head staged in LDS, in 16-byte units:
+//   K   unit (key t, dim octet o) at t * (D / 8) + (o ^ k_swizzle(t))
+//   V^T unit (dim d, key octet c), D = 64 (8 octets):  d * 8 + (c ^ (d & 7))
+//                                  D = 128 (4 octets): d * 4 + (c ^ ((d >> 1) & 3))
 // The swizzles put the eight 16-byte reads that one LDS cycle serves (lanes
 // 8j .. 8j + 7 of an MFMA operand read) on eight different bank groups.
+template <uint32_t kDim>
 struct KvTile {
-    half8_t k[kTileKeys * 8];
-    half8_t v[64 * 8];
+    half8_t k[PrefillDims<kDim>::kTileKeys * (kDim / 8)];
+    half8_t v[kDim * (PrefillDims<kDim>::kTileKeys / 8)];
 };
 
 __device__ inline uint32_t k_swizzle(uint32_t t) { return (t & 3u) | (((t >> 3) & 1u) << 2); }
-__device__ inline uint32_t k_unit(uint32_t t, uint32_t o) { return t * 8u + (o ^ k_swizzle(t)); }
-__device__ inline uint32_t v_unit(uint32_t d, uint32_t c) { return d * 8u + (c ^ (d & 7u)); }
+template <uint32_t kDim>
+__device__ inline uint32_t k_unit(uint32_t t, uint32_t o)
+{
+    return t * (kDim / 8) + (o ^ k_swizzle(t));
+}
+template <uint32_t kDim>
+__device__ inline uint32_t v_unit(uint32_t d, uint32_t c)
+{
+    return kDim == 64 ? d * 8u + (c ^ (d & 7u)) : d * 4u + (c ^ ((d >> 1) & 3u));
+}
 
-// Keys per group-table segment of the prefill kernel (multiple of 64).
+// Keys per group-table segment of the prefill kernel (a multiple of the tile).
 constexpr unsigned kSegmentKeys = 4096;
 constexpr unsigned kSegmentGroups = kSegmentKeys / 8;
 
 // One 8-key group of the segment resolved for the block's layer and KV head:
-// k points at the group's first key in K panel 0 (panel 1, dims 32..63, is
-// kpanel elements further), v at the group's first key in V^T row 0 (dim d is
-// d * vw elements further).
+// k points at the group's first key in K panel 0 (panel p, dims 32 p ..
+// 32 p + 31, is p * kpanel elements further), v at the group's first key in
+// V^T row 0 (dim d is d * vw elements further).
 struct HeadGroup {
     const uint16_t* k;
     const uint16_t* v;
@@ -94,6 +124,7 @@ struct HeadGroup {
 // Records the 8-key groups of [c0, c1) that entry `e` covers, for layer /
 // head.  An entry whose pages do not keep 8-token groups aligned (or that
 // names no page of the storage) switches the block to the generic path.
+template <uint32_t kDim>
 __device__ inline void add_head_groups(const PoolView& P, kimkv_block_desc const& e, uint32_t layer, uint32_t h,
                                        uint32_t c0, uint32_t c1, uint32_t T, HeadGroup* groups, uint32_t* s_generic)
 {
@@ -114,14 +145,15 @@ __device__ inline void add_head_groups(const PoolView& P, kimkv_block_desc const
     uint32_t const vw = v_width(cap);
     for (uint32_t g = (lo - c0) >> 3; g < (hi - c0 + 7) >> 3; ++g) {
         uint32_t const pt0 = c0 + 8 * g - b;
-        groups[g] = HeadGroup{hb + k_offset(cap, 64, pt0, 0), hb + v_offset(cap, 64, pt0, 0), cap * 32u, vw, 0};
+        groups[g] = HeadGroup{hb + k_offset(cap, kDim, pt0, 0), hb + v_offset(cap, kDim, pt0, 0), cap * 32u, vw, 0};
     }
 }
 
 // A thread's share of one tile in flight: two K units and two V^T units.
-//   K unit j:   chunk c = tid + 256 j -> group c / 64, panel (c / 32) % 2, key (c / 4) % 8, octet c % 4
-//               (a wave reads one 8-key group: two contiguous 512-byte runs of the page)
-//   V^T unit j: key octet 4 j + tid % 4, dim tid / 4
+//   K unit j:   chunk c = tid + 256 j -> group c / (D), panel (c / 32) % (D / 32), key (c / 4) % 8, octet c % 4
+//               (a wave reads half or all of one 8-key group: contiguous 512-byte runs of the page)
+//   V^T unit j: D = 64:  key octet 4 j + tid % 4, dim tid / 4
+//               D = 128: key octet tid % 4, dim tid / 4 + 64 j
 //               (four consecutive lanes read one dim row of a 32-key V^T panel: 64 contiguous bytes)
 struct TileLoad {
     half8_t k[2];
@@ -137,21 +169,22 @@ __device__ __attribute__((always_inline)) inline uint64_t uniform_u64(uint64_t x
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
-// kFull: all 64 keys of the tile are below nvalid and every group of the
-// segment names a page, so no lane needs a check.  A K unit's group (c / 64)
-// is the same for the whole wave: its base goes to SGPRs and each lane adds a
-// 32-bit offset (panel (tid / 32) % 2, key (tid / 4) % 8, octet tid % 4, the
+// kFull: all keys of the tile are below nvalid and every group of the segment
+// names a page, so no lane needs a check.  A K unit's group (c / D) is the
+// same for the whole wave: its base goes to SGPRs and each lane adds a 32-bit
+// offset (panel (tid / 32) % (D / 32), key (tid / 4) % 8, octet tid % 4, the
 // same for both units).
-template <bool kFull>
+template <uint32_t kDim, bool kFull>
 __device__ inline void tile_fetch(TileLoad& r, const HeadGroup* groups, uint32_t tg, uint32_t nvalid, uint32_t tid)
 {
+    using Dims = PrefillDims<kDim>;
     half8_t const zero8 = {};
     uint32_t const tk = (tid >> 2) & 7u;
     uint32_t const k_off = tk * 64u + (tid & 3u) * 16u;
-    uint32_t const k_panel = (tid >> 5) & 1u;
+    uint32_t const k_panel = (tid >> 5) & (Dims::kPanels - 1);
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
-        uint32_t const g = (tid >> 6) + kWaves * j;
+        uint32_t const g = (tid + kBlock * j) / kDim;
         if (kFull || 8 * g + tk < nvalid) {
             HeadGroup const e = groups[tg + g];
             uint64_t const kb = uniform_u64(reinterpret_cast<uintptr_t>(e.k));
@@ -163,16 +196,17 @@ __device__ inline void tile_fetch(TileLoad& r, const HeadGroup* groups, uint32_t
         } else {
             r.k[j] = zero8;
         }
-        uint32_t const ko = 4 * j + (tid & 3u);
+        uint32_t const ko = kDim == 64 ? 4 * j + (tid & 3u) : tid & 3u;
+        uint32_t const d = kDim == 64 ? tid >> 2 : (tid >> 2) + 64 * j;
         if (kFull) {
             HeadGroup const e = groups[tg + ko];
-            r.v[j] = load_half8_stream(e.v + (tid >> 2) * e.vw);
+            r.v[j] = load_half8_stream(e.v + d * e.vw);
         } else {
             r.v[j] = zero8;
             if (8 * ko < nvalid) {
                 HeadGroup const e = groups[tg + ko];
                 if (e.v != nullptr) {
-                    r.v[j] = load_half8_stream(e.v + (tid >> 2) * e.vw);
+                    r.v[j] = load_half8_stream(e.v + d * e.vw);
                     if (8 * ko + 8 > nvalid) {
                         uint32_t const keep = nvalid - 8 * ko;
 #pragma unroll
@@ -186,14 +220,20 @@ __device__ inline void tile_fetch(TileLoad& r, const HeadGroup* groups, uint32_t
     }
 }
 
-__device__ inline void tile_store(KvTile& t, const TileLoad& r, uint32_t tid)
+template <uint32_t kDim>
+__device__ inline void tile_store(KvTile<kDim>& t, const TileLoad& r, uint32_t tid)
 {
+    using Dims = PrefillDims<kDim>;
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
         uint32_t const c = tid + kBlock * j;
-        uint32_t const key = 8 * (c >> 6) + ((c >> 2) & 7u);
-        t.k[k_unit(key, 4 * ((c >> 5) & 1u) + (c & 3u))] = r.k[j];
-        t.v[v_unit(tid >> 2, 4 * j + (tid & 3u))] = r.v[j];
+        uint32_t const key = 8 * (c / kDim) + ((c >> 2) & 7u);
+        t.k[k_unit<kDim>(key, 4 * ((c >> 5) & (Dims::kPanels - 1)) + (c & 3u))] = r.k[j];
+        if (kDim == 64) {
+            t.v[v_unit<kDim>(tid >> 2, 4 * j + (tid & 3u))] = r.v[j];
+        } else {
+            t.v[v_unit<kDim>((tid >> 2) + 64 * j, tid & 3u)] = r.v[j];
+        }
     }
 }
 
@@ -213,26 +253,29 @@ __device__ inline float xor32(float v)
 
 // One wave of the fast path: kColBlocks column blocks of 16 columns, each
 // tpw new tokens x the G query heads of KV head h.  S^T = K.Q^T and
-// O^T += V^T.P^T per 64-key tile, with the keys of a 32-key half permuted
+// O^T += V^T.P^T per tile, with the keys of a 32-key half permuted
 // so that the S^T accumulator layout is the P^T operand layout (lane l holds
 // keys 8 (l / 16) .. + 7 of its column).
+template <uint32_t kDim>
 struct PrefillWave {
     uint32_t l, a, r, x;
     uint32_t i0;                       // first new token of the wave
-    half8_t qb[kColBlocks][2];
+    half8_t qb[kColBlocks][PrefillDims<kDim>::kPanels];
     uint32_t limit[kColBlocks];        // last key this lane's column may see
     float scale2;
     float m_run[kColBlocks];
-    // acc[0..3]: O^T dims 16 db .. 16 db + 15; acc[4] row 0: the softmax
-    // denominator, accumulated by the MFMA from a ones row of V^T.
-    float4_t acc[5][kColBlocks];
+    // acc[db], db < kDb: O^T dims 16 db .. 16 db + 15; acc[kDb] row 0: the
+    // softmax denominator, accumulated by the MFMA from a ones row of V^T.
+    float4_t acc[PrefillDims<kDim>::kDb + 1][kColBlocks];
     half8_t ones;
 };
 
-__device__ void prefill_wave_init(PrefillWave& w, const kimkv_prefill_item& item, uint32_t h, PrefillShape shape,
-                                  uint32_t QH, uint32_t i0)
+template <uint32_t kDim>
+__device__ void prefill_wave_init(PrefillWave<kDim>& w, const kimkv_prefill_item& item, uint32_t h,
+                                  PrefillShape shape, uint32_t QH, uint32_t i0)
 {
-    constexpr uint32_t D = 64;
+    constexpr uint32_t D = kDim;
+    using Dims = PrefillDims<kDim>;
     w.l = threadIdx.x & 63u;
     w.a = w.l >> 4;
     w.r = w.l & 15u;
@@ -246,58 +289,64 @@ __device__ void prefill_wave_init(PrefillWave& w, const kimkv_prefill_item& item
         uint32_t const q = h * shape.G + w.r % shape.G;
         bool const valid = i < item.new_tokens;
         w.limit[cb] = T0 + (valid ? i : 0);
-        w.qb[cb][0] = zero8;
-        w.qb[cb][1] = zero8;
+#pragma unroll
+        for (uint32_t p = 0; p < Dims::kPanels; ++p) w.qb[cb][p] = zero8;
         if (valid) {
             const uint16_t* qrow = item.query + (static_cast<uint64_t>(i) * QH + q) * D;
-            w.qb[cb][0] = *reinterpret_cast<const half8_t*>(qrow + w.a * 8);
-            w.qb[cb][1] = *reinterpret_cast<const half8_t*>(qrow + 32 + w.a * 8);
+#pragma unroll
+            for (uint32_t p = 0; p < Dims::kPanels; ++p) {
+                w.qb[cb][p] = *reinterpret_cast<const half8_t*>(qrow + 32 * p + w.a * 8);
+            }
         }
         w.m_run[cb] = -INFINITY;
 #pragma unroll
-        for (uint32_t db = 0; db < 5; ++db) w.acc[db][cb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t db = 0; db <= Dims::kDb; ++db) w.acc[db][cb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
     w.scale2 = item.attention_scale * kLog2e;
     _Float16 const one = static_cast<_Float16>(w.r == 0 ? 1.0f : 0.0f);
     w.ones = half8_t{one, one, one, one, one, one, one, one};
 }
 
-// Keys [t0, t0 + 64) from the staged tile; nvalid = valid keys from t0 on.
-// kMasked: some key of the tile is past nvalid or past a column's limit.
-template <bool kMasked>
-__device__ inline void prefill_wave_step(PrefillWave& w, const KvTile& tile, uint32_t t0, uint32_t nvalid)
+// Keys [t0, t0 + kTileKeys) from the staged tile; nvalid = valid keys from t0
+// on.  kMasked: some key of the tile is past nvalid or past a column's limit.
+template <uint32_t kDim, bool kMasked>
+__device__ inline void prefill_wave_step(PrefillWave<kDim>& w, const KvTile<kDim>& tile, uint32_t t0, uint32_t nvalid)
 {
+    using Dims = PrefillDims<kDim>;
     // Column block 0's scores are issued first, so its softmax (VALU) runs
     // while block 1's score MFMAs execute, and block 1's softmax while block
     // 0's output MFMAs execute.
-    half8_t kop[2][2][2];
+    half8_t kop[Dims::kKB][2][Dims::kPanels];
 #pragma unroll
-    for (uint32_t kb = 0; kb < 2; ++kb) {
+    for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
         for (uint32_t e = 0; e < 2; ++e) {
             uint32_t const t = 32 * kb + 8 * w.x + 4 * e + (w.l & 3u);
-            kop[kb][e][0] = tile.k[k_unit(t, w.a)];
-            kop[kb][e][1] = tile.k[k_unit(t, 4 + w.a)];
+#pragma unroll
+            for (uint32_t p = 0; p < Dims::kPanels; ++p) kop[kb][e][p] = tile.k[k_unit<kDim>(t, 4 * p + w.a)];
         }
     }
-    float4_t s[kColBlocks][2][2];
+    float4_t s[kColBlocks][Dims::kKB][2];
 #pragma unroll
     for (uint32_t cb = 0; cb < kColBlocks; ++cb) {
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
                 float4_t z = {};
-                z = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[kb][e][0], w.qb[cb][0], z, 0, 0, 0);
-                s[cb][kb][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[kb][e][1], w.qb[cb][1], z, 0, 0, 0);
+#pragma unroll
+                for (uint32_t p = 0; p < Dims::kPanels; ++p) {
+                    z = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[kb][e][p], w.qb[cb][p], z, 0, 0, 0);
+                }
+                s[cb][kb][e] = z;
             }
         }
     }
-    half8_t vop[2][4];
+    half8_t vop[Dims::kKB][Dims::kDb];
 #pragma unroll
-    for (uint32_t kb = 0; kb < 2; ++kb) {
+    for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
-        for (uint32_t db = 0; db < 4; ++db) vop[kb][db] = tile.v[v_unit(16 * db + w.r, 4 * kb + w.a)];
+        for (uint32_t db = 0; db < Dims::kDb; ++db) vop[kb][db] = tile.v[v_unit<kDim>(16 * db + w.r, 4 * kb + w.a)];
     }
 #pragma unroll
     for (uint32_t cb = 0; cb < kColBlocks; ++cb) {
@@ -305,7 +354,7 @@ __device__ inline void prefill_wave_step(PrefillWave& w, const KvTile& tile, uin
         // taken on the unscaled dots (scale2 > 0 keeps the order and rounding is monotonic).
         float mx = -INFINITY;
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
 #pragma unroll
@@ -336,42 +385,58 @@ __device__ inline void prefill_wave_step(PrefillWave& w, const KvTile& tile, uin
             float const alpha = grow ? __builtin_amdgcn_exp2f(w.m_run[cb] - m_cand) : 1.0f;
             if (grow) w.m_run[cb] = m_cand;
 #pragma unroll
-            for (uint32_t db = 0; db < 5; ++db) w.acc[db][cb] *= alpha;
+            for (uint32_t db = 0; db <= Dims::kDb; ++db) w.acc[db][cb] *= alpha;
         }
-        float const mref = w.m_run[cb];
-        bool const empty = kMasked && mref == -INFINITY;
-        half8_t pb[2];
+        // kSplitP: a column without a finite score yet takes 0 for its
+        // reference, so its weights 2^-inf are zeros without a test of each.
+        float const mref = !Dims::kSplitP ? w.m_run[cb]
+            : w.m_run[cb] == -INFINITY ? 0.0f : w.m_run[cb] - Dims::kWeightShift;
+        bool const empty = !Dims::kSplitP && kMasked && mref == -INFINITY;
+        half8_t pb[Dims::kKB];
+        half8_t pl[Dims::kKB];
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
             for (uint32_t e = 0; e < 2; ++e) {
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i) {
                     float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[cb][kb][e][i], w.scale2, -mref));
-                    if (kMasked && empty) p = 0.0f;
-                    pb[kb][4 * e + i] = static_cast<_Float16>(p);
+                    if (!Dims::kSplitP && kMasked && empty) p = 0.0f;
+                    _Float16 const hi = static_cast<_Float16>(p);
+                    pb[kb][4 * e + i] = hi;
+                    if (Dims::kSplitP) pl[kb][4 * e + i] = static_cast<_Float16>(p - static_cast<float>(hi));
                 }
             }
         }
 #pragma unroll
-        for (uint32_t kb = 0; kb < 2; ++kb) {
+        for (uint32_t kb = 0; kb < Dims::kKB; ++kb) {
 #pragma unroll
-            for (uint32_t db = 0; db < 4; ++db) {
+            for (uint32_t db = 0; db < Dims::kDb; ++db) {
                 w.acc[db][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[kb][db], pb[kb], w.acc[db][cb], 0, 0, 0);
+                if (Dims::kSplitP) {
+                    w.acc[db][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[kb][db], pl[kb], w.acc[db][cb], 0, 0, 0);
+                }
             }
-            w.acc[4][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w.ones, pb[kb], w.acc[4][cb], 0, 0, 0);
+            w.acc[Dims::kDb][cb] =
+                __builtin_amdgcn_mfma_f32_16x16x32_f16(w.ones, pb[kb], w.acc[Dims::kDb][cb], 0, 0, 0);
+            if (Dims::kSplitP) {
+                w.acc[Dims::kDb][cb] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_f16(w.ones, pl[kb], w.acc[Dims::kDb][cb], 0, 0, 0);
+            }
         }
     }
 }
 
-__device__ void prefill_wave_store(PrefillWave& w, const kimkv_prefill_item& item, uint32_t h, PrefillShape shape,
-                                   uint32_t QH)
+template <uint32_t kDim>
+__device__ void prefill_wave_store(PrefillWave<kDim>& w, const kimkv_prefill_item& item, uint32_t h,
+                                   PrefillShape shape, uint32_t QH)
 {
-    constexpr uint32_t D = 64;
+    constexpr uint32_t D = kDim;
+    constexpr uint32_t kDb = PrefillDims<kDim>::kDb;
 #pragma unroll
     for (uint32_t cb = 0; cb < kColBlocks; ++cb) {
-        // Row 0 of acc[4] (element 0 on lanes 0..15) is the denominator; the other lanes hold zeros.
-        float l_tot = w.acc[4][cb][0] + xor16(w.acc[4][cb][0]);
+        // Row 0 of acc[kDb] (element 0 on lanes 0..15) is the denominator; the other lanes hold zeros.
+        float l_tot = w.acc[kDb][cb][0] + xor16(w.acc[kDb][cb][0]);
         l_tot += xor32(l_tot);
         uint32_t const i = w.i0 + cb * shape.tpw + w.r / shape.G;
         if (i >= item.new_tokens) continue;
@@ -379,7 +444,7 @@ __device__ void prefill_wave_store(PrefillWave& w, const kimkv_prefill_item& ite
         float const inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         uint16_t* out = item.output + (static_cast<uint64_t>(i) * QH + q) * D;
 #pragma unroll
-        for (uint32_t db = 0; db < 4; ++db) {
+        for (uint32_t db = 0; db < kDb; ++db) {
             uint32_t lo = static_cast<uint32_t>(__half_as_ushort(__float2half_rn(w.acc[db][cb][0] * inv)))
                 | (static_cast<uint32_t>(__half_as_ushort(__float2half_rn(w.acc[db][cb][1] * inv))) << 16);
             uint32_t hi = static_cast<uint32_t>(__half_as_ushort(__float2half_rn(w.acc[db][cb][2] * inv)))
@@ -478,14 +543,18 @@ __device__ void prefill_row_generic(const PoolView& P, const kimkv_prefill_item&
 
 // Either order != nullptr (an ordered launch: dispatch index -> XCD-logical
 // index -> order entry) or block_prefix != nullptr (head-major blocks, the
-// blocks of an item from its last tokens to its first).
+// blocks of an item from its last tokens to its first).  kDim: the head dim
+// of the MFMA path (64 or 128); a storage of another head dim runs the
+// kDim = 64 instance's generic path.
+template <uint32_t kDim>
 __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const kimkv_prefill_item* items,
                                                             const uint32_t* block_prefix,
                                                             const kimkv_prefill_block* order, uint32_t item_count,
                                                             uint32_t total_blocks, uint32_t QH)
 {
     __shared__ HeadGroup groups[kSegmentGroups];
-    __shared__ KvTile tiles[2];
+    constexpr uint32_t kTileKeys = PrefillDims<kDim>::kTileKeys;
+    __shared__ KvTile<kDim> tiles[2];
     __shared__ GenericScratch scratch[kWaves];
     __shared__ uint32_t s_item;
     __shared__ uint32_t s_generic;
@@ -538,10 +607,16 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
     uint32_t const last = min(i_block + per_block, item.new_tokens) - 1;
     uint32_t const kend = T0 + last + 1;
 
-    if (shape.mfma) {
+    // What the generic path takes and the MFMA path would not: a scale that
+    // does not keep the order of the scores, rows below the vectors'
+    // alignment (head dim 64 has always required both).
+    bool const general = kDim == 128
+        && (!(item.attention_scale > 0.0f) || (reinterpret_cast<uintptr_t>(item.query) & 15u) != 0
+            || (reinterpret_cast<uintptr_t>(item.output) & 7u) != 0);
+    if (shape.mfma && D == kDim && !general) {
         uint32_t const wave_tokens = kColBlocks * shape.tpw;
         uint32_t const i0 = i_block + wave * wave_tokens;
-        PrefillWave w;
+        PrefillWave<kDim> w;
         prefill_wave_init(w, item, h, shape, QH, i0);
         bool const wave_has_rows = i0 < item.new_tokens;
         // Keys up to the wave's last token (exclusive end) and its first token's limit.
@@ -554,7 +629,7 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
             __syncthreads();
             uint32_t const idx0 = find_descriptor_wave(item.descriptors, item.descriptor_count, s0);
             for (uint32_t j = tid; j <= ngroups && idx0 + j < item.descriptor_count; j += kBlock) {
-                add_head_groups(P, item.descriptors[idx0 + j], item.layer, h, s0, s1, item.token_count, groups,
+                add_head_groups<kDim>(P, item.descriptors[idx0 + j], item.layer, h, s0, s1, item.token_count, groups,
                                 &s_generic);
             }
             __syncthreads();
@@ -571,21 +646,21 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
             // Tile j is computed from tiles[j % 2] while tile j + 1 sits in the
             // other register set and tile j + 2's loads are issued: each tile's
             // loads have two compute phases to land.
-            auto compute = [&](const KvTile& tile, uint32_t j) {
+            auto compute = [&](const KvTile<kDim>& tile, uint32_t j) {
                 uint32_t const t0 = s0 + j * kTileKeys;
                 if (t0 >= wave_kend) return;
                 if (t0 + kTileKeys <= s1 && t0 + kTileKeys <= wave_full) {
-                    prefill_wave_step<false>(w, tile, t0, s1 - t0);
+                    prefill_wave_step<kDim, false>(w, tile, t0, s1 - t0);
                 } else {
-                    prefill_wave_step<true>(w, tile, t0, s1 - t0);
+                    prefill_wave_step<kDim, true>(w, tile, t0, s1 - t0);
                 }
             };
             auto fetch = [&](TileLoad& ld, uint32_t j) {
                 uint32_t const nvalid = s1 - s0 - j * kTileKeys;
                 if (!holes && nvalid >= kTileKeys) {
-                    tile_fetch<true>(ld, groups, j * (kTileKeys / 8), nvalid, tid);
+                    tile_fetch<kDim, true>(ld, groups, j * (kTileKeys / 8), nvalid, tid);
                 } else {
-                    tile_fetch<false>(ld, groups, j * (kTileKeys / 8), nvalid, tid);
+                    tile_fetch<kDim, false>(ld, groups, j * (kTileKeys / 8), nvalid, tid);
                 }
             };
             TileLoad la, lb;
@@ -620,6 +695,21 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
     }
 }
 
+void launch_prefill(const kimkv_storage* storage, dim3 grid, const kimkv_prefill_item* items,
+                    const uint32_t* block_prefix, const kimkv_prefill_block* order, uint32_t item_count,
+                    uint32_t total_blocks, uint32_t query_heads, kimkv_stream_t stream)
+{
+    auto go = [&](auto kernel) {
+        kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), items, block_prefix, order, item_count,
+                                                    total_blocks, query_heads);
+    };
+    if (storage->layout.head_dim == 128) {
+        go(prefill_kernel<128>);
+    } else {
+        go(prefill_kernel<64>);
+    }
+}
+
 }  // namespace
 }  // namespace kimkv
 
@@ -650,8 +740,8 @@ kimkv_status kimkv_paged_prefill_batch(const kimkv_storage* storage, const kimkv
     dim3 const grid(total_blocks * storage->layout.kv_heads);
     void* start = nullptr;
     kernel_timing_begin(TimedKernel::Prefill, native(stream), &start);
-    prefill_kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_items, device_block_prefix,
-                                                        nullptr, item_count, total_blocks, query_heads);
+    launch_prefill(storage, grid, device_items, device_block_prefix, nullptr, item_count, total_blocks, query_heads,
+                   stream);
     kimkv_status const st = launch_status();
     kernel_timing_end(TimedKernel::Prefill, native(stream), start);
     return st;
@@ -758,8 +848,8 @@ kimkv_status kimkv_paged_prefill_ordered(const kimkv_storage* storage, const kim
     if (order_count == 0 || item_count == 0) return KIMKV_OK;
     void* start = nullptr;
     kernel_timing_begin(TimedKernel::Prefill, native(stream), &start);
-    prefill_kernel<<<order_count, kBlock, 0, native(stream)>>>(pool_view(*storage), device_items, nullptr,
-                                                               device_order, item_count, 1u, query_heads);
+    launch_prefill(storage, dim3(order_count), device_items, nullptr, device_order, item_count, 1u, query_heads,
+                   stream);
     kimkv_status const st = launch_status();
     kernel_timing_end(TimedKernel::Prefill, native(stream), start);
     return st;
