@@ -9,6 +9,8 @@
 //   gatherKernel                       src/cuda/kv/page_kernels.cu:184-242
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_common.h"
 #include "runtime_internal.h"
 
@@ -26,37 +28,91 @@ struct TokEntry {
     uint32_t pt;
 };
 
-// Resolves tokens [t0, t0+n) (n <= 64) of a table into LDS entries.  Tokens
-// not covered by a valid descriptor get page == nullptr.  All threads of the
-// block must call it.
-__device__ void build_tile_table(const PoolView& P, const kimkv_block_desc* desc, uint32_t count,
-                                 uint32_t t0, uint32_t n, TokEntry* tab, uint32_t* s_idx)
+// x / d and x % d for a d that is uniform over the launch: the reciprocal is
+// computed on the host (floor((2^32 - 1) / d)), so the quotient is at most one
+// short and one compare corrects it.  Exact for every x < 2^32; an integer
+// division by a kernel argument is about 30 instructions, this is 7.
+struct Divisor {
+    uint32_t d;
+    uint32_t m;
+};
+inline Divisor divisor(uint32_t d) { return Divisor{d, 0xFFFFFFFFu / (d == 0 ? 1u : d)}; }
+
+__device__ inline uint32_t div_mod(uint32_t x, Divisor v, uint32_t* rem)
 {
-    uint32_t const tid = threadIdx.x;
-    if (tid < kTile) {
-        tab[tid].page = nullptr;
-        uint32_t const idx = find_descriptor_wave(desc, count, t0);
-        if (tid == 0) {
-            *s_idx = idx;
+    uint32_t q = __umulhi(x, v.m);
+    uint32_t r = x - q * v.d;
+    if (r >= v.d) {
+        ++q;
+        r -= v.d;
+    }
+    *rem = r;
+    return q;
+}
+
+// Entries of one wave's table read: lane i holds entry idx + i; token lane of
+// the tile is resolved from the entry that covers it.  Returns whether entry
+// idx covers t0 (then the following 63 cover everything the tile can reach).
+__device__ inline bool resolve_tile_wave(const PoolView& P, const kimkv_block_desc* desc, uint32_t count, uint32_t idx,
+                                         uint32_t t0, uint32_t n, bool need_hit, TokEntry* tab)
+{
+    uint32_t const lane = threadIdx.x & (kWave - 1);
+    uint32_t lo = 0;
+    uint32_t hi = 0;
+    uint32_t begin = 0;
+    uint32_t cap = 0;
+    uint64_t page = 0;
+    bool hit = false;
+    if (lane < n && idx + lane < count) {
+        kimkv_block_desc const e = desc[idx + lane];
+        begin = e.logical_token_begin;
+        hit = begin <= t0 && t0 - begin < e.valid_tokens;
+        lo = max(begin, t0);
+        hi = min(begin + e.valid_tokens, t0 + n);
+        cap = e.page_token_capacity;
+        if (lo < hi && e.valid_tokens <= cap) {
+            page = reinterpret_cast<uint64_t>(page_base(P, e.kind, e.slot, cap));
         }
     }
-    __syncthreads();
-    uint32_t const idx = *s_idx;
-    // At most n descriptors overlap the tile, starting at idx.
-    if (tid < n && idx + tid < count) {
-        kimkv_block_desc const e = desc[idx + tid];
-        uint32_t const b = e.logical_token_begin;
-        uint32_t const end = b + e.valid_tokens;
-        uint32_t const lo = max(b, t0);
-        uint32_t const hi = min(end, t0 + n);
-        if (lo < hi && e.valid_tokens <= e.page_token_capacity) {
-            uint16_t* page = page_base(P, e.kind, e.slot, e.page_token_capacity);
-            if (page != nullptr) {
-                for (uint32_t t = lo; t < hi; ++t) {
-                    tab[t - t0] = TokEntry{page, e.page_token_capacity, t - b};
-                }
-            }
+    bool const found = (__ballot(hit) & 1u) != 0;
+    if (need_hit && !found) return false;
+    // readlane returns a signed word: made unsigned before it is widened.
+    auto from = [](uint32_t v, int j) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), j)); };
+    auto const page_lo = static_cast<uint32_t>(page);
+    auto const page_hi = static_cast<uint32_t>(page >> 32);
+    TokEntry mine{nullptr, 0, 0};
+    for (uint64_t left = __ballot(page != 0); left != 0; left &= left - 1) {
+        int const j = __ffsll(static_cast<unsigned long long>(left)) - 1;
+        uint32_t const jlo = from(lo, j);
+        uint32_t const jhi = from(hi, j);
+        uint64_t const jpage = static_cast<uint64_t>(from(page_lo, j)) | static_cast<uint64_t>(from(page_hi, j)) << 32;
+        uint32_t const jcap = from(cap, j);
+        uint32_t const jbegin = from(begin, j);
+        if (t0 + lane >= jlo && t0 + lane < jhi) {
+            mine = TokEntry{reinterpret_cast<uint16_t*>(jpage), jcap, t0 + lane - jbegin};
         }
+    }
+    if (lane < n) tab[lane] = mine;
+    return found;
+}
+
+// Resolves tokens [t0, t0+n) (n <= 64) of a table into LDS entries.  Tokens
+// not covered by a valid descriptor get page == nullptr.  All threads of the
+// block must call it.  The first entry is guessed before it is searched for:
+// t0 / 64 when every entry before it is a full extent page, t0 / 8 when they
+// are full micro pages; each guess is one wave's single read of the table,
+// and a guess counts only if its first entry covers t0.
+__device__ void build_tile_table(const PoolView& P, const kimkv_block_desc* desc, uint32_t count,
+                                 uint32_t t0, uint32_t n, TokEntry* tab, uint32_t* s_hit)
+{
+    uint32_t const wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) *s_hit = 0;
+    __syncthreads();
+    if (wave < 2 && resolve_tile_wave(P, desc, count, t0 / (wave == 0 ? 64u : 8u), t0, n, true, tab)) *s_hit = 1;
+    __syncthreads();
+    if (*s_hit == 0 && wave == 0) {
+        uint32_t const idx = find_descriptor_wave(desc, count, t0);
+        static_cast<void>(resolve_tile_wave(P, desc, count, idx, t0, n, false, tab));
     }
     __syncthreads();
 }
@@ -64,8 +120,64 @@ __device__ void build_tile_table(const PoolView& P, const kimkv_block_desc* desc
 // ---------------------------------------------------------------------------
 // Batched append: one block per (job, layer).
 // ---------------------------------------------------------------------------
+// Stores the first `count` (<= 8) halves of v at a 16-byte aligned address.
+__device__ inline void store_prefix(uint16_t* p, u32x4_t v, uint32_t count)
+{
+    if (count >= 8) {
+        *reinterpret_cast<u32x4_t*>(p) = v;
+        return;
+    }
+    uint32_t at = 0;
+    if (count & 4u) {
+        *reinterpret_cast<uint2*>(p) = make_uint2(v[0], v[1]);
+        at = 4;
+    }
+    if (count & 2u) {
+        *reinterpret_cast<uint32_t*>(p + at) = at == 4 ? v[2] : v[0];
+        at += 2;
+    }
+    if (count & 1u) p[at] = static_cast<uint16_t>(at < 4 ? (at == 2 ? v[1] : v[0]) : (at == 6 ? v[3] : v[2]));
+}
+
+struct AppendDivisors {
+    Divisor hd;        // H * D
+    Divisor hd8;       // H * D / 8
+    Divisor d;         // D
+    Divisor d8;        // D / 8
+};
+
+// Copies tokens [0, n) of a page's blocks of one layer to another page, K in
+// pieces of 8 dims and V^T in pieces of 8 tokens of one dim, of which the last
+// piece stores only the copied tokens (its page may hold others' bytes past
+// them).  A thread loads one piece of each before it stores either: more of
+// them in flight costs registers that the long appends of this kernel need
+// for waves (batches of four: 107 registers, a prompt's append of 5448 tokens
+// x 22 layers 57 us instead of 40).  Element by element the copy was seven
+// dependent rounds for a 7-token tail of 4 heads x 64; the append of 64 lanes
+// x 22 layers, a quarter of the tails copied, went from 12.6 to 7.7 us.
+// Both capacities and D are multiples of 8; src and dst are the layer's blocks.
+__device__ inline void copy_tokens_wide(const AppendDivisors& dv, uint32_t n, const uint16_t* src, uint32_t scap,
+                                        uint16_t* dst, uint32_t dcap)
+{
+    uint32_t const D = dv.d.d;
+    uint32_t const kchunks = n * dv.hd8.d;
+    uint32_t const vchunks = (n + 7) / 8 * dv.hd.d;
+    for (uint32_t i = threadIdx.x; i < max(kchunks, vchunks); i += kBlock) {
+        uint32_t rem, c, d;
+        uint32_t const t = div_mod(i, dv.hd8, &rem);
+        uint32_t const kh = div_mod(rem, dv.d8, &c);
+        uint32_t const g = div_mod(i, dv.hd, &rem);
+        uint32_t const vh = div_mod(rem, dv.d, &d);
+        u32x4_t k, v;
+        if (i < kchunks) k = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * kh + k_offset(scap, D, t, c * 8));
+        if (i < vchunks) v = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * vh + v_offset(scap, D, g * 8, d));
+        if (i < kchunks) *reinterpret_cast<u32x4_t*>(dst + 2 * dcap * D * kh + k_offset(dcap, D, t, c * 8)) = k;
+        if (i < vchunks) store_prefix(dst + 2 * dcap * D * vh + v_offset(dcap, D, g * 8, d), v, n - g * 8);
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_append_job* jobs,
-                                                        uint32_t job_count)
+                                                        uint32_t job_count, AppendDivisors dv)
 {
     if (blockIdx.x >= job_count) return;
     kimkv_append_job const job = jobs[blockIdx.x];
@@ -83,24 +195,28 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
     }
     uint32_t const tid = threadIdx.x;
 
+    // The copied positions lie below the written ones: neither waits for the other.
     if (job.cow_tokens != 0) {
         uint32_t const scap = pool_tokens(P, job.cow_kind);
         uint16_t const* src = page_base(P, job.cow_kind, job.cow_slot, scap);
         uint32_t const n = job.cow_tokens;
         if (src != nullptr && n <= scap && n <= dcap && n <= job.dst_token) {
-            uint32_t const per_head = n * D;
-            for (uint32_t i = tid; i < H * per_head; i += kBlock) {
-                uint32_t const h = i / per_head;
-                uint32_t const rem = i - h * per_head;
-                uint32_t const t = rem / D;
-                uint32_t const d = rem - t * D;
-                uint64_t const sh = head_block(P, scap, layer, h);
-                uint64_t const dh = head_block(P, dcap, layer, h);
-                dst[dh + k_offset(dcap, D, t, d)] = src[sh + k_offset(scap, D, t, d)];
-                dst[dh + v_offset(dcap, D, t, d)] = src[sh + v_offset(scap, D, t, d)];
+            if (((D | scap | dcap) & 7u) == 0) {
+                copy_tokens_wide(dv, n, src + head_block(P, scap, layer, 0), scap, dst + head_block(P, dcap, layer, 0), dcap);
+            } else {
+                uint32_t const per_head = n * D;
+                for (uint32_t i = tid; i < H * per_head; i += kBlock) {
+                    uint32_t const h = i / per_head;
+                    uint32_t const rem = i - h * per_head;
+                    uint32_t const t = rem / D;
+                    uint32_t const d = rem - t * D;
+                    uint64_t const sh = head_block(P, scap, layer, h);
+                    uint64_t const dh = head_block(P, dcap, layer, h);
+                    dst[dh + k_offset(dcap, D, t, d)] = src[sh + k_offset(scap, D, t, d)];
+                    dst[dh + v_offset(dcap, D, t, d)] = src[sh + v_offset(scap, D, t, d)];
+                }
             }
         }
-        __syncthreads();
     }
 
     uint32_t const HD = H * D;
@@ -113,13 +229,11 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         && ((reinterpret_cast<uintptr_t>(sk) | reinterpret_cast<uintptr_t>(sv)) & 15u) == 0;
     if (src_aligned) {
         // K: 16-byte pieces of 8 dims of one token (contiguous in source and page).
-        uint32_t const dchunks = D / 8;
-        uint32_t const kchunks = job.token_count * H * dchunks;
+        uint32_t const kchunks = job.token_count * dv.hd8.d;
         for (uint32_t i = tid; i < kchunks; i += kBlock) {
-            uint32_t const t = i / (H * dchunks);
-            uint32_t const rem = i - t * (H * dchunks);
-            uint32_t const h = rem / dchunks;
-            uint32_t const dc = rem - h * dchunks;
+            uint32_t rem, dc;
+            uint32_t const t = div_mod(i, dv.hd8, &rem);
+            uint32_t const h = div_mod(rem, dv.d8, &dc);
             u32x4_t const v = *reinterpret_cast<const u32x4_t*>(sk + static_cast<uint64_t>(t) * stride + h * D + dc * 8);
             *reinterpret_cast<u32x4_t*>(dst + head_block(P, dcap, layer, h)
                                         + k_offset(dcap, D, job.dst_token + t, dc * 8)) = v;
@@ -130,10 +244,9 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         if (v_groups) {
             uint32_t const vchunks = (job.token_count / 8) * HD;
             for (uint32_t i = tid; i < vchunks; i += kBlock) {
-                uint32_t const g = i / HD;
-                uint32_t const r = i - g * HD;
-                uint32_t const h = r / D;
-                uint32_t const d = r - h * D;
+                uint32_t r, d;
+                uint32_t const g = div_mod(i, dv.hd, &r);
+                uint32_t const h = div_mod(r, dv.d, &d);
                 const uint16_t* src = sv + static_cast<uint64_t>(8 * g) * stride + r;
                 u32x4_t w;
 #pragma unroll
@@ -147,10 +260,9 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
             return;
         }
         for (uint32_t i = tid; i < total; i += kBlock) {
-            uint32_t const t = i / HD;
-            uint32_t const rem = i - t * HD;
-            uint32_t const h = rem / D;
-            uint32_t const d = rem - h * D;
+            uint32_t rem, d;
+            uint32_t const t = div_mod(i, dv.hd, &rem);
+            uint32_t const h = div_mod(rem, dv.d, &d);
             dst[head_block(P, dcap, layer, h) + v_offset(dcap, D, job.dst_token + t, d)] =
                 sv[static_cast<uint64_t>(t) * stride + rem];
         }
@@ -170,19 +282,22 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
 }
 
 // ---------------------------------------------------------------------------
-// Gather: block = (64-token tile, group of layers); output [L][2][T][H][D].
-// Fast path (full tile whose 8-token groups each sit 8-aligned in one page,
-// D % 8 == 0): every thread issues all its 16-byte non-temporal loads before
-// any store.  K rows are copied straight; V^T is transposed through LDS
-// (16-byte chunks of 8 tokens of one dim row in, 16-byte chunks of 8 dims of
-// one token out; the chunk column is XOR-swizzled by the token's group so the
-// scattered 2-byte writes of one instruction spread over the banks).  Other
-// tiles take the element-wise path.
+// Gather: block = (64-token tile, group of layers, block of kRows columns of
+// the H * D row); output [L][2][T][H][D].  Fast path (every 8-token group of
+// the tile sits 8-aligned in one page, D % 8 == 0): a thread issues all its
+// 16-byte non-temporal loads, K and V^T, before any store.  K rows are copied
+// straight; V^T is transposed through LDS (16-byte chunks of 8 tokens of one
+// dim row in, 16-byte chunks of 8 dims of one token out; the chunk column is
+// XOR-swizzled by the token's group so the scattered 2-byte writes of one
+// instruction spread over the banks).  A tile of fewer than 64 tokens and a
+// last block of fewer columns take it too: loads past the edge repeat the
+// last token or column, stores past it are left out (the last group's load
+// reads the page's own positions past the tile).  Other tiles take the
+// element-wise path.  Bound by HBM when the chip is full (5.6 TB/s read and
+// written at 16384 tokens x 22 layers), by the chain of table read, load and
+// store when it is not (560..2021 tokens x 22 layers, last tile partial: 10
+// and 20 us; 42 us with that tile copied 2 bytes at a time).
 // ---------------------------------------------------------------------------
-constexpr unsigned kRowChunk = 256;            // V rows (head x dim) per pass
-constexpr unsigned kStageRow = kRowChunk + 8;  // u16 per staged token row (16-byte multiple)
-constexpr unsigned kGatherLoads = 8;           // 16-byte loads in flight per thread
-
 typedef const __attribute__((address_space(1))) u32x4_t global_u32x4_t;
 typedef __attribute__((address_space(1))) u32x4_t global_u32x4_out_t;
 
@@ -201,126 +316,59 @@ __device__ inline uint32_t stage_col(uint32_t t, uint32_t r)
     return (((r >> 3) ^ ((t >> 3) & 3u)) << 3) | (r & 7u);
 }
 
-// K rows of one (tile, layer): straight 16-byte copies, all loads first.
-__device__ inline void gather_k_fast(const PoolView& P, const TokEntry* tab, uint32_t layer, uint16_t* out_base)
+// Columns [r0, r0 + kRows) of one (tile, layer).  n tokens, `cols` valid columns.
+template <uint32_t kRows, bool kWhole>
+__device__ inline void gather_kv_fast(const PoolView& P, const TokEntry* tab, uint32_t layer, uint32_t r0, uint32_t n,
+                                      uint32_t cols, Divisor dim, uint16_t* k_base, uint16_t* v_base, uint16_t* stage)
 {
-    uint32_t const tid = threadIdx.x;
-    uint32_t const D = P.dim;
-    uint32_t const dchunks = D / 8;
-    uint32_t const per_token = P.heads * dchunks;
-    uint32_t const total = kTile * per_token;
-    for (uint32_t base = 0; base < total; base += kBlock * kGatherLoads) {
-        u32x4_t v[kGatherLoads];
-#pragma unroll
-        for (uint32_t k = 0; k < kGatherLoads; ++k) {
-            uint32_t const i = base + k * kBlock + tid;
-            if (i < total) {
-                uint32_t const t = i / per_token;
-                uint32_t const c = i - t * per_token;
-                uint32_t const h = c / dchunks;
-                TokEntry const e = tab[t];
-                v[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, (c - h * dchunks) * 8));
-            }
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kGatherLoads; ++k) {
-            uint32_t const i = base + k * kBlock + tid;
-            if (i < total) store16_nt(out_base + static_cast<uint64_t>(i) * 8, v[k]);
-        }
-    }
-}
-
-// V^T rows of one (tile, layer) transposed through LDS.
-__device__ inline void gather_v_fast(const PoolView& P, const TokEntry* tab, uint32_t layer, uint16_t* out_base,
-                                     uint16_t* stage)
-{
+    constexpr uint32_t kStageRow = kRows + 8;                 // u16 per staged token row (16-byte multiple)
+    constexpr uint32_t per = kTile * kRows / 8 / kBlock;      // 16-byte chunks per thread, each of K and V
+    constexpr uint32_t per_token = kRows / 8;
     uint32_t const tid = threadIdx.x;
     uint32_t const D = P.dim;
     uint32_t const HD = P.heads * D;
-    for (uint32_t r0 = 0; r0 < HD; r0 += kRowChunk) {
-        uint32_t const rows = min(kRowChunk, HD - r0);
-        uint32_t const chunks = rows * 8;   // (row, 8-token group) pairs
-        // Chunk q: group (q & 3) + 4 * ((q >> 2) / rows), row (q >> 2) % rows: four consecutive
-        // lanes read one 64-byte dim row of a 32-token V^T panel.
-        for (uint32_t base = 0; base < chunks; base += kBlock * kGatherLoads) {
-            u32x4_t v[kGatherLoads];
-#pragma unroll
-            for (uint32_t k = 0; k < kGatherLoads; ++k) {
-                uint32_t const q = base + k * kBlock + tid;
-                if (q < chunks) {
-                    uint32_t const rr = (q >> 2) % rows;
-                    uint32_t const g = (q & 3u) + 4u * ((q >> 2) / rows);
-                    uint32_t const r = r0 + rr;
-                    uint32_t const h = r / D;
-                    TokEntry const e = tab[8 * g];
-                    v[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, r - h * D));
-                }
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kGatherLoads; ++k) {
-                uint32_t const q = base + k * kBlock + tid;
-                if (q < chunks) {
-                    uint32_t const rr = (q >> 2) % rows;
-                    uint32_t const g = (q & 3u) + 4u * ((q >> 2) / rows);
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; ++j) {
-                        uint32_t const t = 8 * g + j;
-                        uint32_t const word = v[k][j >> 1];
-                        stage[t * kStageRow + stage_col(t, rr)] =
-                            static_cast<uint16_t>((j & 1u) ? (word >> 16) : (word & 0xFFFFu));
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        uint32_t const per_token = rows / 8;
-        for (uint32_t i = tid; i < kTile * per_token; i += kBlock) {
-            uint32_t const t = i / per_token;
-            uint32_t const c = i - t * per_token;
-            u32x4_t const w = *reinterpret_cast<const u32x4_t*>(&stage[t * kStageRow + stage_col(t, c * 8)]);
-            store16_nt(out_base + static_cast<uint64_t>(t) * HD + r0 + c * 8, w);
-        }
-        __syncthreads();
-    }
-}
-
-// One (tile, layer) with H * D == kRowChunk: the K and V^T loads of the
-// layer (8 + 8 per thread) are all in flight before the first store.
-__device__ inline void gather_kv_fast(const PoolView& P, const TokEntry* tab, uint32_t layer, uint16_t* k_base,
-                                      uint16_t* v_base, uint16_t* stage)
-{
-    constexpr uint32_t rows = kRowChunk;
-    constexpr uint32_t per = kTile * rows / 8 / kBlock;   // 16-byte chunks per thread, each of K and V
-    uint32_t const tid = threadIdx.x;
-    uint32_t const D = P.dim;
-    uint32_t const dchunks = D / 8;
-    constexpr uint32_t per_token = rows / 8;
     u32x4_t kv[per], vv[per];
 #pragma unroll
     for (uint32_t k = 0; k < per; ++k) {
         uint32_t const i = k * kBlock + tid;
-        uint32_t const t = i / per_token;
-        uint32_t const c = i - t * per_token;
-        uint32_t const h = c / dchunks;
+        uint32_t t = i / per_token;
+        uint32_t c = i % per_token * 8;
+        if (!kWhole) {
+            t = min(t, n - 1);
+            c = min(c, cols - 8);
+        }
+        uint32_t d;
+        uint32_t const h = div_mod(r0 + c, dim, &d);
         TokEntry const e = tab[t];
-        kv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, (c - h * dchunks) * 8));
+        kv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, d));
+    }
+    // Chunk q: four consecutive lanes read one 64-byte dim row of a 32-token V^T panel.
+#pragma unroll
+    for (uint32_t k = 0; k < per; ++k) {
+        uint32_t const q = k * kBlock + tid;
+        uint32_t rr = (q >> 2) % kRows;
+        uint32_t t = 8 * ((q & 3u) + 4u * ((q >> 2) / kRows));
+        if (!kWhole) {
+            t = min(t, (n - 1) & ~7u);
+            rr = min(rr, cols - 1);
+        }
+        uint32_t d;
+        uint32_t const h = div_mod(r0 + rr, dim, &d);
+        TokEntry const e = tab[t];
+        vv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, d));
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < per; ++k) {
+        uint32_t const i = k * kBlock + tid;
+        uint32_t const t = i / per_token;
+        uint32_t const c = i % per_token * 8;
+        if (kWhole || (t < n && c < cols)) store16_nt(k_base + static_cast<uint64_t>(t) * HD + r0 + c, kv[k]);
     }
 #pragma unroll
     for (uint32_t k = 0; k < per; ++k) {
         uint32_t const q = k * kBlock + tid;
-        uint32_t const rr = (q >> 2) % rows;
-        uint32_t const g = (q & 3u) + 4u * ((q >> 2) / rows);
-        uint32_t const h = rr / D;
-        TokEntry const e = tab[8 * g];
-        vv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, rr - h * D));
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < per; ++k) store16_nt(k_base + static_cast<uint64_t>(k * kBlock + tid) * 8, kv[k]);
-#pragma unroll
-    for (uint32_t k = 0; k < per; ++k) {
-        uint32_t const q = k * kBlock + tid;
-        uint32_t const rr = (q >> 2) % rows;
-        uint32_t const g = (q & 3u) + 4u * ((q >> 2) / rows);
+        uint32_t const rr = (q >> 2) % kRows;
+        uint32_t const g = (q & 3u) + 4u * ((q >> 2) / kRows);
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
             uint32_t const t = 8 * g + j;
@@ -333,65 +381,72 @@ __device__ inline void gather_kv_fast(const PoolView& P, const TokEntry* tab, ui
     for (uint32_t k = 0; k < per; ++k) {
         uint32_t const i = k * kBlock + tid;
         uint32_t const t = i / per_token;
-        uint32_t const c = i - t * per_token;
-        u32x4_t const w = *reinterpret_cast<const u32x4_t*>(&stage[t * kStageRow + stage_col(t, c * 8)]);
-        store16_nt(v_base + static_cast<uint64_t>(t) * rows + c * 8, w);
+        uint32_t const c = i % per_token * 8;
+        if (kWhole || (t < n && c < cols)) {
+            u32x4_t const w = *reinterpret_cast<const u32x4_t*>(&stage[t * kStageRow + stage_col(t, c)]);
+            store16_nt(v_base + static_cast<uint64_t>(t) * HD + r0 + c, w);
+        }
     }
     __syncthreads();
 }
 
-// Block = (64-token tile, group of layers_per_block layers): the tile's page
-// table is resolved once for all its layers and both components.
+// The tile's page table is resolved once for all the block's layers and both
+// components.
+template <uint32_t kRows>
 __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_block_desc* desc,
                                                         uint32_t count, uint32_t T, uint32_t layers_per_block,
-                                                        uint16_t* out)
+                                                        Divisor dim, uint16_t* out)
 {
     __shared__ TokEntry tab[kTile];
-    __shared__ uint32_t s_idx;
-    __shared__ __align__(16) uint16_t stage[kTile * kStageRow];
+    __shared__ uint32_t s_hit;
+    __shared__ __align__(16) uint16_t stage[kTile * (kRows + 8)];
 
     uint32_t const t0 = blockIdx.x * kTile;
     uint32_t const n = min(kTile, T - t0);
-    build_tile_table(P, desc, count, t0, n, tab, &s_idx);
+    build_tile_table(P, desc, count, t0, n, tab, &s_hit);
 
     uint32_t const D = P.dim;
     uint32_t const HD = P.heads * D;
     uint32_t const tid = threadIdx.x;
     uint32_t const l0 = blockIdx.y * layers_per_block;
     uint32_t const l1 = min(P.layers, l0 + layers_per_block);
+    uint32_t const r0 = blockIdx.z * kRows;
+    uint32_t const cols = min(kRows, HD - r0);
 
     int group_ok = 1;
-    if (tid < kTile / 8) {
+    if (8 * tid < n) {
+        uint32_t const last = min(n, 8 * tid + 8) - 1;
         TokEntry const a = tab[8 * tid];
-        TokEntry const b = tab[8 * tid + 7];
-        group_ok = a.page != nullptr && b.page == a.page && (a.pt & 7u) == 0 && b.pt == a.pt + 7
+        TokEntry const b = tab[last];
+        group_ok = a.page != nullptr && b.page == a.page && (a.pt & 7u) == 0 && b.pt == a.pt + (last - 8 * tid)
             && (a.cap & 7u) == 0;
     }
-    bool const fast = __syncthreads_and(group_ok) && n == kTile && (D & 7u) == 0;
+    bool const fast = __syncthreads_and(group_ok) && (D & 7u) == 0;
+    bool const whole = n == kTile && cols == kRows;
 
     for (uint32_t layer = l0; layer < l1; ++layer) {
         uint16_t* k_base = out + (static_cast<uint64_t>(layer * 2) * T + t0) * HD;
         uint16_t* v_base = out + (static_cast<uint64_t>(layer * 2 + 1) * T + t0) * HD;
-        if (fast && HD == kRowChunk) {
-            gather_kv_fast(P, tab, layer, k_base, v_base, stage);
+        if (fast && whole) {
+            gather_kv_fast<kRows, true>(P, tab, layer, r0, n, cols, dim, k_base, v_base, stage);
             continue;
         }
         if (fast) {
-            gather_k_fast(P, tab, layer, k_base);
-            gather_v_fast(P, tab, layer, v_base, stage);
+            gather_kv_fast<kRows, false>(P, tab, layer, r0, n, cols, dim, k_base, v_base, stage);
             continue;
         }
-        // Element-wise path: partial tiles, unaligned groups, D % 8 != 0.
-        for (uint32_t i = tid; i < n * HD; i += kBlock) {
-            uint32_t const t = i / HD;
-            uint32_t const r = i - t * HD;
+        // Element-wise path: groups across pages or off the 8-token grid, unmapped tokens, D % 8 != 0.
+        for (uint32_t i = tid; i < n * cols; i += kBlock) {
+            uint32_t const t = i / cols;
+            uint32_t const r = r0 + i - t * cols;
             TokEntry const e = tab[t];
             if (e.page == nullptr) continue;
-            uint32_t const h = r / D;
-            uint32_t const d = r - h * D;
+            uint32_t d;
+            uint32_t const h = div_mod(r, dim, &d);
             uint16_t const* hb = e.page + head_block(P, e.cap, layer, h);
-            k_base[i] = hb[k_offset(e.cap, D, e.pt, d)];
-            v_base[i] = hb[v_offset(e.cap, D, e.pt, d)];
+            uint64_t const at = static_cast<uint64_t>(t) * HD + r;
+            k_base[at] = hb[k_offset(e.cap, D, e.pt, d)];
+            v_base[at] = hb[v_offset(e.cap, D, e.pt, d)];
         }
     }
 }
@@ -485,12 +540,12 @@ __global__ __launch_bounds__(kBlock) void fill_table_kernel(PoolView P, const ki
                                                             uint32_t stream_id)
 {
     __shared__ TokEntry tab[kTile];
-    __shared__ uint32_t s_idx;
+    __shared__ uint32_t s_hit;
     uint32_t const t0 = token_begin + blockIdx.x * kTile;
     uint32_t const n = min(kTile, token_end - t0);
     uint32_t const layer = blockIdx.y;
     uint32_t const comp = blockIdx.z;
-    build_tile_table(P, desc, count, t0, n, tab, &s_idx);
+    build_tile_table(P, desc, count, t0, n, tab, &s_hit);
     uint32_t const D = P.dim;
     uint32_t const HD = P.heads * D;
     uint32_t const tid = threadIdx.x;
@@ -575,6 +630,15 @@ __global__ __launch_bounds__(kBlock) void fill_kv_kernel(uint16_t* out, uint32_t
 
 using namespace kimkv;
 
+namespace {
+AppendDivisors append_divisors(const kimkv_storage& s)
+{
+    uint32_t const D = s.layout.head_dim;
+    uint32_t const HD = s.layout.kv_heads * D;
+    return AppendDivisors{divisor(HD), divisor(HD / 8), divisor(D), divisor(D / 8)};
+}
+}  // namespace
+
 extern "C" {
 
 kimkv_status kimkv_append_batch(const kimkv_storage* storage, const kimkv_append_job* device_jobs,
@@ -586,7 +650,8 @@ kimkv_status kimkv_append_batch(const kimkv_storage* storage, const kimkv_append
     dim3 const grid(job_count, max_layer_count);
     void* start = nullptr;
     kernel_timing_begin(TimedKernel::Append, native(stream), &start);
-    append_kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_jobs, job_count);
+    append_kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_jobs, job_count,
+                                                         append_divisors(*storage));
     kimkv_status const status = launch_status();
     kernel_timing_end(TimedKernel::Append, native(stream), start);
     return status;
@@ -600,15 +665,30 @@ kimkv_status kimkv_gather(const kimkv_storage* storage, const kimkv_block_desc* 
         || descriptor_count == 0 || total_tokens == 0) {
         return KIMKV_INVALID_ARGUMENT;
     }
-    // Enough workgroups to fill the chip (~8 per CU) with as few table
-    // resolutions as possible: layers are grouped per workgroup.
     uint32_t const tiles = ceil_div(total_tokens, kTile);
     uint32_t const L = storage->layout.layers;
-    uint32_t per = 1;
-    while (per < L && static_cast<uint64_t>(tiles) * ceil_div(L, per * 2) >= 2048) per *= 2;
-    dim3 const grid(tiles, ceil_div(L, per));
-    gather_kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_descriptors,
-                                                       descriptor_count, total_tokens, per, device_output);
+    uint32_t const HD = storage->layout.kv_heads * storage->layout.head_dim;
+    Divisor const dim = divisor(storage->layout.head_dim);
+    auto launch = [&](auto rows) {
+        constexpr uint32_t kRows = decltype(rows)::value;
+        uint32_t const columns = ceil_div(HD, kRows);
+        // Enough workgroups to fill the chip (~8 per CU) with as few table
+        // resolutions as possible: layers are grouped per workgroup.
+        uint32_t per = 1;
+        while (per < L && static_cast<uint64_t>(tiles) * columns * ceil_div(L, per * 2) >= 2048) per *= 2;
+        dim3 const grid(tiles, ceil_div(L, per), columns);
+        gather_kernel<kRows><<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_descriptors,
+                                                                  descriptor_count, total_tokens, per, dim,
+                                                                  device_output);
+    };
+    // 256 columns a block where that fills the chip twice over (16384 tokens x
+    // 22 layers: 128 us, 135 us with 128 columns), narrower blocks where it
+    // does not: more of them share the work (560 tokens x 22 layers: 8.4 us).
+    if (HD > 128 && static_cast<uint64_t>(tiles) * L * ceil_div(HD, 256) >= 512) {
+        launch(std::integral_constant<uint32_t, 256>{});
+    } else {
+        launch(std::integral_constant<uint32_t, 128>{});
+    }
     return launch_status();
 }
 

@@ -65,6 +65,64 @@ def test_append_gather_bit_exact(dev, shape, T):
     assert np.array_equal(got, pools.gather(table, T))
 
 
+@pytest.mark.parametrize("layout", ["hetero", "micro", "ragged"])
+@pytest.mark.parametrize("shape", [(2, 4, 64), (2, 1, 64), (1, 3, 128), (1, 1, 8), (1, 2, 12)])
+def test_gather_tile_edges_bit_exact(dev, shape, layout):
+    """Tiles of 1..64 tokens and rows that are no multiple of a column block
+    (64, 384, 8 and 24 dims); "ragged" tables start their pages off the
+    8-token grid and leave one token unmapped, whose output stays as it was."""
+    L, H, D = shape
+    for T in (1, 7, 8, 9, 33, 63, 64, 65, 71, 129):
+        print(f"gather {layout} L={L} H={H} D={D} T={T}", flush=True)
+        storage = dev.Storage(L, H, D, 64, 8)
+        pools = oracle.HostPools(L, H, D, 64, 8)
+        alloc = helpers.SlotAllocator(64, 8, seed=T)
+        if layout == "hetero":
+            table = helpers.hetero_table(T, alloc)
+        elif layout == "micro":
+            table = helpers.uniform_table(T, 8, alloc)
+        else:
+            entries, at = [], 0
+            while at < T:
+                n = min(T - at, 3 if not entries else 8)
+                entries.append((alloc.take(helpers.MICRO), 1, at, n, 8, 0))
+                at += n + (len(entries) == 2)
+            table = np.array(entries, dtype=helpers.DESC)
+        inp = _input(L, H, D, T, seed=T)
+        _populate(dev, storage, pools, table, inp)
+        want = np.full((L, 2, T, H * D), 0x1234, dtype=np.uint16)
+        for e in table:
+            span = slice(int(e["logical_token_begin"]), int(e["logical_token_begin"]) + int(e["valid_tokens"]))
+            want[:, :, span] = inp.reshape(L, 2, T, H * D)[:, :, span]
+        out = dev.upload(np.full(want.size + 64, 0x1234, dtype=np.uint16))
+        desc = dev.upload(table)
+        dev.check(dev.lib().kimkv_gather(storage.h, desc.ptr, len(table), T, out.ptr, None), "gather")
+        got = dev.download(out.ptr, (want.size + 64,), np.uint16)
+        assert np.array_equal(got[:want.size], want.reshape(-1))
+        assert np.all(got[want.size:] == 0x1234)
+
+
+@pytest.mark.parametrize("shape", [(4, 64), (1, 8), (8, 128), (3, 12)])
+def test_cow_counts_keep_other_tokens(dev, shape):
+    """A copied tail of every length: the copied and the new token land, and
+    the destination page's later tokens keep their bytes."""
+    H, D = shape
+    storage = dev.Storage(1, H, D, 32, 4)
+    pools = oracle.HostPools(1, H, D, 32, 4)
+    table = np.array([(s, 1, 8 * s, 8, 8, 0) for s in range(16)], dtype=helpers.DESC)
+    inp = _input(1, H, D, 128, seed=9)
+    _populate(dev, storage, pools, table, inp)
+    new_kv = oracle.synth_rows(8 * 2 * H * D, 321, 0, H * D).reshape(8, 2, H * D)
+    buf = dev.upload(new_kv)
+    jobs = np.zeros(7, dtype=dev.APPEND_JOB)
+    for n in range(1, 8):   # page n -> page 8 + n, n tokens copied, token n written
+        jobs[n - 1] = (buf.ptr + 4 * n * H * D, buf.ptr + 4 * n * H * D + 2 * H * D, 0, 0, 0, 1, 1, 8 + n, n, n, n, 0, 0)
+        pools.copy_layer_tokens(0, n, 0, 8 + n, n, 0)
+        pools.write_layer_token(0, 8 + n, n, 0, new_kv[n, 0], new_kv[n, 1])
+    storage.append_batch(jobs)
+    assert np.array_equal(storage.gather(table, 128), pools.gather(table, 128))
+
+
 def test_patch_descriptors(dev):
     """kimkv_patch_descriptors: whole-table writes (one longer than a
     workgroup's 256 words) and one-entry tail patches land exactly on their
