@@ -147,18 +147,17 @@ __device__ inline uint64_t head_block(const PoolView& p, uint32_t cap, uint32_t 
 __host__ __device__ inline uint32_t k_width(uint32_t D) { return D % 32u == 0u ? 32u : D; }
 __host__ __device__ inline uint32_t v_width(uint32_t cap) { return cap % 32u == 0u ? 32u : cap; }
 
-// Offsets inside a block fit 32 bits (a layer's block of one page).  d < D and
-// t < cap, so the column block is a shift or 0: a division by the width, which
-// the compiler cannot see to be 32 or the whole row, costs about 30
-// instructions in kernels that copy 16 bytes per offset.
-__host__ __device__ inline uint32_t k_offset(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
+__host__ __device__ inline uint64_t k_offset(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
 {
-    return D % 32u == 0u ? (d >> 5) * cap * 32u + t * 32u + (d & 31u) : t * D + d;
+    uint32_t const kw = k_width(D);
+    return static_cast<uint64_t>(d / kw) * cap * kw + static_cast<uint64_t>(t) * kw + d % kw;
 }
 
-__host__ __device__ inline uint32_t v_offset(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
+__host__ __device__ inline uint64_t v_offset(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
 {
-    return cap * D + (cap % 32u == 0u ? (t >> 5) * D * 32u + d * 32u + (t & 31u) : d * cap + t);
+    uint32_t const vw = v_width(cap);
+    return static_cast<uint64_t>(cap) * D + static_cast<uint64_t>(t / vw) * D * vw + static_cast<uint64_t>(d) * vw
+        + t % vw;
 }
 
 // ---- XCD-aware workgroup order ----------------------------------------------

@@ -50,6 +50,21 @@ __device__ inline uint32_t div_mod(uint32_t x, Divisor v, uint32_t* rem)
     return q;
 }
 
+// k_offset and v_offset (device_common.h) in 32 bits and without their
+// divisions: d < D and t < cap, so the column block is a shift or 0, which
+// the compiler cannot tell of a width that is 32 or the whole row.  A copy
+// computes two such offsets for 16 bytes; the attention kernels, which
+// compute few, are 4% slower with this form (a branch per operand load).
+__device__ inline uint32_t k_at(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
+{
+    return D % 32u == 0u ? (d >> 5) * cap * 32u + t * 32u + (d & 31u) : t * D + d;
+}
+
+__device__ inline uint32_t v_at(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
+{
+    return cap * D + (cap % 32u == 0u ? (t >> 5) * D * 32u + d * 32u + (t & 31u) : d * cap + t);
+}
+
 // Entries of one wave's table read: lane i holds entry idx + i; token lane of
 // the tile is resolved from the entry that covers it.  Returns whether entry
 // idx covers t0 (then the following 63 cover everything the tile can reach).
@@ -169,10 +184,10 @@ __device__ inline void copy_tokens_wide(const AppendDivisors& dv, uint32_t n, co
         uint32_t const g = div_mod(i, dv.hd, &rem);
         uint32_t const vh = div_mod(rem, dv.d, &d);
         u32x4_t k, v;
-        if (i < kchunks) k = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * kh + k_offset(scap, D, t, c * 8));
-        if (i < vchunks) v = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * vh + v_offset(scap, D, g * 8, d));
-        if (i < kchunks) *reinterpret_cast<u32x4_t*>(dst + 2 * dcap * D * kh + k_offset(dcap, D, t, c * 8)) = k;
-        if (i < vchunks) store_prefix(dst + 2 * dcap * D * vh + v_offset(dcap, D, g * 8, d), v, n - g * 8);
+        if (i < kchunks) k = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * kh + k_at(scap, D, t, c * 8));
+        if (i < vchunks) v = *reinterpret_cast<const u32x4_t*>(src + 2 * scap * D * vh + v_at(scap, D, g * 8, d));
+        if (i < kchunks) *reinterpret_cast<u32x4_t*>(dst + 2 * dcap * D * kh + k_at(dcap, D, t, c * 8)) = k;
+        if (i < vchunks) store_prefix(dst + 2 * dcap * D * vh + v_at(dcap, D, g * 8, d), v, n - g * 8);
     }
 }
 
@@ -212,8 +227,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
                     uint32_t const d = rem - t * D;
                     uint64_t const sh = head_block(P, scap, layer, h);
                     uint64_t const dh = head_block(P, dcap, layer, h);
-                    dst[dh + k_offset(dcap, D, t, d)] = src[sh + k_offset(scap, D, t, d)];
-                    dst[dh + v_offset(dcap, D, t, d)] = src[sh + v_offset(scap, D, t, d)];
+                    dst[dh + k_at(dcap, D, t, d)] = src[sh + k_at(scap, D, t, d)];
+                    dst[dh + v_at(dcap, D, t, d)] = src[sh + v_at(scap, D, t, d)];
                 }
             }
         }
@@ -236,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
             uint32_t const h = div_mod(rem, dv.d8, &dc);
             u32x4_t const v = *reinterpret_cast<const u32x4_t*>(sk + static_cast<uint64_t>(t) * stride + h * D + dc * 8);
             *reinterpret_cast<u32x4_t*>(dst + head_block(P, dcap, layer, h)
-                                        + k_offset(dcap, D, job.dst_token + t, dc * 8)) = v;
+                                        + k_at(dcap, D, job.dst_token + t, dc * 8)) = v;
         }
         // V^T: 16-byte pieces of 8 tokens of one dim when the tokens sit in
         // 8-aligned groups of the page, else one element at a time.
@@ -255,7 +270,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
                         | (static_cast<uint32_t>(src[static_cast<uint64_t>(2 * j + 1) * stride]) << 16);
                 }
                 *reinterpret_cast<u32x4_t*>(dst + head_block(P, dcap, layer, h)
-                                            + v_offset(dcap, D, job.dst_token + 8 * g, d)) = w;
+                                            + v_at(dcap, D, job.dst_token + 8 * g, d)) = w;
             }
             return;
         }
@@ -263,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
             uint32_t rem, d;
             uint32_t const t = div_mod(i, dv.hd, &rem);
             uint32_t const h = div_mod(rem, dv.d, &d);
-            dst[head_block(P, dcap, layer, h) + v_offset(dcap, D, job.dst_token + t, d)] =
+            dst[head_block(P, dcap, layer, h) + v_at(dcap, D, job.dst_token + t, d)] =
                 sv[static_cast<uint64_t>(t) * stride + rem];
         }
         return;
@@ -276,8 +291,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         uint64_t const so = layer_off + static_cast<uint64_t>(t) * job.src_token_stride + rem;
         uint64_t const dh = head_block(P, dcap, layer, h);
         uint32_t const pt = job.dst_token + t;
-        dst[dh + k_offset(dcap, D, pt, d)] = job.src_key[so];
-        dst[dh + v_offset(dcap, D, pt, d)] = job.src_value[so];
+        dst[dh + k_at(dcap, D, pt, d)] = job.src_key[so];
+        dst[dh + v_at(dcap, D, pt, d)] = job.src_value[so];
     }
 }
 
@@ -340,7 +355,7 @@ __device__ inline void gather_kv_fast(const PoolView& P, const TokEntry* tab, ui
         uint32_t d;
         uint32_t const h = div_mod(r0 + c, dim, &d);
         TokEntry const e = tab[t];
-        kv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, d));
+        kv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + k_at(e.cap, D, e.pt, d));
     }
     // Chunk q: four consecutive lanes read one 64-byte dim row of a 32-token V^T panel.
 #pragma unroll
@@ -355,7 +370,7 @@ __device__ inline void gather_kv_fast(const PoolView& P, const TokEntry* tab, ui
         uint32_t d;
         uint32_t const h = div_mod(r0 + rr, dim, &d);
         TokEntry const e = tab[t];
-        vv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, d));
+        vv[k] = load16_nt(e.page + head_block(P, e.cap, layer, h) + v_at(e.cap, D, e.pt, d));
     }
 #pragma unroll
     for (uint32_t k = 0; k < per; ++k) {
@@ -445,8 +460,8 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_
             uint32_t const h = div_mod(r, dim, &d);
             uint16_t const* hb = e.page + head_block(P, e.cap, layer, h);
             uint64_t const at = static_cast<uint64_t>(t) * HD + r;
-            k_base[at] = hb[k_offset(e.cap, D, e.pt, d)];
-            v_base[at] = hb[v_offset(e.cap, D, e.pt, d)];
+            k_base[at] = hb[k_at(e.cap, D, e.pt, d)];
+            v_base[at] = hb[v_at(e.cap, D, e.pt, d)];
         }
     }
 }
@@ -500,8 +515,8 @@ __global__ __launch_bounds__(kBlock) void promote_kernel(PoolView P, const kimkv
             uint32_t const t = rem / dchunks;
             uint32_t const dc = rem - t * dchunks;
             uint4 const v = *reinterpret_cast<uint4 const*>(
-                src[t >> 3] + head_block(P, mt, layer, h) + k_offset(mt, D, t & 7u, dc * 8));
-            *reinterpret_cast<uint4*>(dst + head_block(P, et, layer, h) + k_offset(et, D, t, dc * 8)) = v;
+                src[t >> 3] + head_block(P, mt, layer, h) + k_at(mt, D, t & 7u, dc * 8));
+            *reinterpret_cast<uint4*>(dst + head_block(P, et, layer, h) + k_at(et, D, t, dc * 8)) = v;
         }
         // V^T: (h, d, k) -- micro row d (8 tokens, 16 bytes) -> extent row d at 8k.
         uint32_t const vchunks = H * D * 8;
@@ -511,8 +526,8 @@ __global__ __launch_bounds__(kBlock) void promote_kernel(PoolView P, const kimkv
             uint32_t const d = rem / 8;
             uint32_t const k = rem & 7u;
             uint4 const v = *reinterpret_cast<uint4 const*>(
-                src[k] + head_block(P, mt, layer, h) + v_offset(mt, D, 0, d));
-            *reinterpret_cast<uint4*>(dst + head_block(P, et, layer, h) + v_offset(et, D, 8 * k, d)) = v;
+                src[k] + head_block(P, mt, layer, h) + v_at(mt, D, 0, d));
+            *reinterpret_cast<uint4*>(dst + head_block(P, et, layer, h) + v_at(et, D, 8 * k, d)) = v;
         }
         return;
     }
@@ -526,8 +541,8 @@ __global__ __launch_bounds__(kBlock) void promote_kernel(PoolView P, const kimkv
         uint32_t const st = t % mt;
         uint64_t const sh = head_block(P, mt, layer, h);
         uint64_t const dh = head_block(P, et, layer, h);
-        dst[dh + k_offset(et, D, t, d)] = s[sh + k_offset(mt, D, st, d)];
-        dst[dh + v_offset(et, D, t, d)] = s[sh + v_offset(mt, D, st, d)];
+        dst[dh + k_at(et, D, t, d)] = s[sh + k_at(mt, D, st, d)];
+        dst[dh + v_at(et, D, t, d)] = s[sh + v_at(mt, D, st, d)];
     }
 }
 
@@ -558,7 +573,7 @@ __global__ __launch_bounds__(kBlock) void fill_table_kernel(PoolView P, const ki
             if (e.page == nullptr) continue;
             uint32_t const h = r / D;
             uint32_t const d = r - h * D;
-            e.page[head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, d)] =
+            e.page[head_block(P, e.cap, layer, h) + k_at(e.cap, D, e.pt, d)] =
                 synth_f16(seed, kv_row(stream_id, layer, 0, t0 + t), r);
         }
         return;
@@ -583,13 +598,13 @@ __global__ __launch_bounds__(kBlock) void fill_table_kernel(PoolView P, const ki
                 uint32_t const hi = synth_f16(seed, kv_row(stream_id, layer, 1, t0 + tb + 2 * j + 1), r);
                 w[j] = lo | (hi << 16);
             }
-            *reinterpret_cast<uint4*>(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, d)) =
+            *reinterpret_cast<uint4*>(e.page + head_block(P, e.cap, layer, h) + v_at(e.cap, D, e.pt, d)) =
                 make_uint4(w[0], w[1], w[2], w[3]);
         } else {
             for (uint32_t t = tb; t < te; ++t) {
                 TokEntry const f = tab[t];
                 if (f.page == nullptr) continue;
-                f.page[head_block(P, f.cap, layer, h) + v_offset(f.cap, D, f.pt, d)] =
+                f.page[head_block(P, f.cap, layer, h) + v_at(f.cap, D, f.pt, d)] =
                     synth_f16(seed, kv_row(stream_id, layer, 1, t0 + t), r);
             }
         }
