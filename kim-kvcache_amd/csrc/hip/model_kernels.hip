@@ -1,7 +1,7 @@
 // model_kernels.hip -- the dense side of a TinyLlama forward for gfx950:
 // embedding gather, RMSNorm, RoPE (fused with the q / k / v split), SwiGLU,
-// greedy argmax, seeded weight initialisation, and the linear layers on
-// rocBLAS (fp16 in, fp32 accumulate).
+// greedy argmax, seeded weight initialisation, and the linear layers (fp16
+// in, fp32 accumulate): few rows on the kernel below, the rest on hipBLASLt.
 //
 // Counterparts: src/cuda/model/kernels.cuh:11-119 (launchEmbeddingBatch,
 // launchRmsNormBatch, launchRopeBatch, launchResidualAddBatch,
@@ -17,6 +17,7 @@
 #include <cmath>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <unordered_map>
 
 #include "device_common.h"
@@ -234,6 +235,185 @@ __global__ __launch_bounds__(kBlock) void argmax_kernel(const float* logits, uin
     }
 }
 
+// ---------------------------------------------------------------------------
+// Linear layer of up to 64 rows: y[r][n] = sum_k x[r][k] w[n][k] (+ beta y[r][n]).
+// ---------------------------------------------------------------------------
+// Bound by the weights' bytes, so the shape of the work follows them: a
+// workgroup owns kNT 16-feature tiles and 16 kMT rows for the whole sum, its
+// eight waves an eighth of K each.  A wave takes 64 of K a step: 8 lanes read 128 contiguous
+// bytes of a row (in the operand order, where consecutive lanes hold
+// different rows, the loads run at a quarter of the rate), turn them into
+// operand order in LDS of its own, so no wave waits for another, and has the
+// next kDepth steps in flight.  The eight partial tiles are summed in LDS in
+// a fixed order.  Against the library's best of 16 (a call costs it 10 us of
+// host work), K x features, 1 and 64 rows: 2048 x 2048 4.6 and 4.9 us (11.4
+// and 11.2), 5632 x 2048 7.0 and 11.4 us (11.4 and 17.3); 1 row, 2048 x 11264
+// 11.8 us (15.1; 3.9 TB/s of weights), 2048 x 32000 27.1 us (32.0).
+constexpr unsigned kLinearWaves = 8;
+constexpr unsigned kLinearBlock = 64 * kLinearWaves;
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+template <uint32_t kMT, uint32_t kNT>
+__global__ __launch_bounds__(kLinearBlock) void linear_kernel(const uint16_t* x, uint32_t rows, uint32_t K,
+                                                              const uint16_t* w, uint32_t N, void* y, uint32_t y_f32,
+                                                              float beta)
+{
+    constexpr uint32_t kDepth = kMT * kNT == 1 ? 4 : 2;   // steps in flight
+    constexpr uint32_t kPieces = 2 * (kNT + kMT);         // 16-byte pieces a lane reads of a step: weights, then x
+    constexpr uint32_t kStage = kPieces * 64;             // 16-byte units of a wave's step: 128 bytes a row
+    constexpr uint32_t kPart = kMT * kNT * 64;            // and of its partial tiles
+    __shared__ float4_t shared[kLinearWaves * (kStage > kPart ? kStage : kPart)];
+    uint32_t const tid = threadIdx.x;
+    uint32_t const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t const l = tid & 63u;
+    uint32_t const r = l & 15u;
+    uint32_t const a = l >> 4;
+    uint32_t const n0 = blockIdx.x * 16 * kNT;
+    uint32_t const m0 = blockIdx.y * 16 * kMT;
+
+    // Rows and features past the end repeat the last one; their sums are not stored.
+    uint32_t const lr = l >> 3;
+    uint32_t const lc = l & 7u;
+    const half8_t* from[kPieces];
+#pragma unroll
+    for (uint32_t p = 0; p < kPieces; ++p) {
+        const uint16_t* row = p < 2 * kNT ? w + static_cast<uint64_t>(min(n0 + 8 * p + lr, N - 1)) * K
+                                          : x + static_cast<uint64_t>(min(m0 + 8 * (p - 2 * kNT) + lr, rows - 1)) * K;
+        from[p] = reinterpret_cast<const half8_t*>(row) + lc;
+    }
+    uint32_t const steps = K / 64;
+    uint32_t const s0 = steps * wave / kLinearWaves;
+    uint32_t const s1 = steps * (wave + 1) / kLinearWaves;
+    float4_t acc[kNT][kMT] = {};
+    struct Step {
+        half8_t piece[kPieces];
+    };
+    auto load = [&](Step& o, uint32_t s) {
+        s = min(s, s1 - 1);   // a step past the last repeats it: a load without a branch
+#pragma unroll
+        for (uint32_t p = 0; p < kPieces; ++p) o.piece[p] = from[p][8 * s];
+    };
+    // Unit (row, octet c) sits at row * 8 + (c ^ row % 8): both the writes
+    // (8 lanes one row) and the operand reads (8 lanes 8 rows) touch all banks.
+    half8_t* const mine = reinterpret_cast<half8_t*>(shared) + wave * kStage;
+    auto multiply = [&](Step const& o) {
+#pragma unroll
+        for (uint32_t p = 0; p < kPieces; ++p) mine[(8 * p + lr) * 8 + (lc ^ lr)] = o.piece[p];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (uint32_t k = 0; k < 2; ++k) {
+            uint32_t const at = r * 8 + ((4 * k + a) ^ (r & 7u));
+            half8_t xo[kMT];
+#pragma unroll
+            for (uint32_t m = 0; m < kMT; ++m) xo[m] = mine[128 * (kNT + m) + at];
+#pragma unroll
+            for (uint32_t n = 0; n < kNT; ++n) {
+                half8_t const wo = mine[128 * n + at];
+#pragma unroll
+                for (uint32_t m = 0; m < kMT; ++m) {
+                    acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wo, xo[m], acc[n][m], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    if (s0 < s1) {
+        Step ring[kDepth];
+#pragma unroll
+        for (uint32_t i = 0; i < kDepth; ++i) load(ring[i], s0 + i);
+        uint32_t s = s0;
+        for (; s + kDepth < s1; s += kDepth) {
+#pragma unroll
+            for (uint32_t i = 0; i < kDepth; ++i) {
+                multiply(ring[i]);
+                load(ring[i], s + kDepth + i);
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kDepth; ++i) {
+            if (s + i < s1) multiply(ring[i]);
+        }
+    }
+    __syncthreads();   // every wave is done with its steps' space
+    float4_t (*const part)[kNT * kMT][64] = reinterpret_cast<float4_t (*)[kNT * kMT][64]>(shared);
+#pragma unroll
+    for (uint32_t n = 0; n < kNT; ++n) {
+#pragma unroll
+        for (uint32_t m = 0; m < kMT; ++m) part[wave][n * kMT + m][l] = acc[n][m];
+    }
+    __syncthreads();
+    for (uint32_t t = wave; t < kNT * kMT; t += kLinearWaves) {
+        float4_t sum = part[0][t][l];
+#pragma unroll
+        for (uint32_t v = 1; v < kLinearWaves; ++v) sum += part[v][t][l];
+        // Lane (a, r) holds features 4 a .. 4 a + 3 of row r.
+        uint32_t const n = n0 + t / kMT * 16 + 4 * a;
+        uint32_t const row = m0 + t % kMT * 16 + r;
+        if (row >= rows) continue;
+        uint64_t const at = static_cast<uint64_t>(row) * N + n;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            if (n + i >= N) break;
+            if (y_f32 != 0) {
+                float* o = static_cast<float*>(y) + at + i;
+                *o = beta != 0.0f ? sum[i] + beta * *o : sum[i];
+            } else {
+                uint16_t* o = static_cast<uint16_t*>(y) + at + i;
+                *o = f2h(beta != 0.0f ? sum[i] + beta * h2f(*o) : sum[i]);
+            }
+        }
+    }
+}
+
+// What the kernel above takes: whole steps of 64, 16-byte vectors of x and w,
+// and few enough rows for the features.  Every workgroup reads its rows whole, so
+// the more workgroups the features make, the fewer rows pay: one tile a
+// workgroup up to 64 rows (5632 x 2048: 11.4 us, 17.3 in the library), up to
+// three up to 32 (2048 x 11264, 32 rows: 13.2 against 15.0; 60 rows 16.2
+// against 15.0 of GPU time), any number up to 16 (32000 features, 16 rows:
+// 28.8 against 32.0; 64 rows 39 against 33).
+bool linear_fits(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* w, uint32_t out)
+{
+    uint32_t const most = out <= 256 * 16 ? 64 : out <= 768 * 16 ? 32 : 16;
+    return rows <= most && in % 64 == 0
+        && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;
+}
+
+void linear_launch(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* w, uint32_t out, void* y, bool f32,
+                   float beta, hipStream_t stream)
+{
+    // One workgroup per CU: as many feature tiles each as that takes, up to
+    // four, or the rows in two blocks where that still fits (the second
+    // block, on the same XCD when the tiles are a multiple of 8, reads the
+    // weights from its L2: 5632 x 2048, 64 rows, 16.8 us as one, 11.4 as two).
+    uint32_t const tiles = (out + 15) / 16;
+    uint32_t const halves = rows > 16 && tiles <= 128 ? 2 : 1;
+    uint32_t const block_rows = (rows + halves - 1) / halves;
+    auto go = [&](auto mt, auto nt) {
+        constexpr uint32_t kMT = decltype(mt)::value;
+        constexpr uint32_t kNT = decltype(nt)::value;
+        dim3 const grid((tiles + kNT - 1) / kNT, (rows + 16 * kMT - 1) / (16 * kMT));
+        linear_kernel<kMT, kNT><<<grid, kLinearBlock, 0, stream>>>(x, rows, in, w, out, y, f32 ? 1u : 0u, beta);
+    };
+    auto features = [&](auto mt) {
+        if (tiles <= 256) go(mt, std::integral_constant<uint32_t, 1>{});
+        else if (tiles <= 512) go(mt, std::integral_constant<uint32_t, 2>{});
+        else if (tiles <= 768) go(mt, std::integral_constant<uint32_t, 3>{});
+        else go(mt, std::integral_constant<uint32_t, 4>{});
+    };
+    if (block_rows <= 16) features(std::integral_constant<uint32_t, 1>{});
+    else if (block_rows > 32) go(std::integral_constant<uint32_t, 4>{}, std::integral_constant<uint32_t, 1>{});
+    else if (tiles <= 256) go(std::integral_constant<uint32_t, 2>{}, std::integral_constant<uint32_t, 1>{});
+    else if (tiles <= 512) go(std::integral_constant<uint32_t, 2>{}, std::integral_constant<uint32_t, 2>{});
+    else go(std::integral_constant<uint32_t, 2>{}, std::integral_constant<uint32_t, 3>{});
+}
+
 unsigned grid_for(uint64_t count)
 {
     uint64_t const b = (count + kBlock - 1) / kBlock;
@@ -267,6 +447,7 @@ struct LtKeyHash {
 };
 
 struct LtPlan {
+    bool own{false};   // linear_kernel, where the call's addresses allow it
     hipblasLtMatmulDesc_t desc{nullptr};
     hipblasLtMatrixLayout_t a{nullptr}, b{nullptr}, c{nullptr};
     hipblasLtMatmulAlgo_t algo{};
@@ -452,7 +633,12 @@ kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features
     if (ctx == nullptr) return KIMKV_RUNTIME_UNAVAILABLE;
     LtKey const key{rows, in_features, out_features, static_cast<uint8_t>(y_f32 != 0), static_cast<uint8_t>(beta != 0.0f)};
     auto it = ctx->plans.find(key);
+    bool const fits = linear_fits(x, rows, in_features, weight, out_features);
     if (it == ctx->plans.end()) {
+        if (fits) {
+            linear_launch(x, rows, in_features, weight, out_features, y, y_f32 != 0, beta, native(stream));
+            return launch_status();
+        }
         LtPlan p;
         hipblasLtMatmulHeuristicResult_t cand[1];
         if (!lt_describe(key, p)) return KIMKV_RUNTIME_UNAVAILABLE;
@@ -462,6 +648,10 @@ kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features
         }
         p.algo = cand[0].algo;
         it = ctx->plans.emplace(key, p).first;
+    }
+    if (it->second.own && fits) {
+        linear_launch(x, rows, in_features, weight, out_features, y, y_f32 != 0, beta, native(stream));
+        return launch_status();
     }
     hipblasStatus_t const r = lt_run(st, *ctx, it->second, it->second.algo, x, weight, y, beta, native(stream));
     return r == HIPBLAS_STATUS_SUCCESS ? KIMKV_OK : KIMKV_SUBMISSION_FAILED;
@@ -495,19 +685,33 @@ kimkv_status kimkv_linear_tune(const uint16_t* x, uint32_t rows, uint32_t in_fea
         lt_destroy(p);
         return n < 1 ? KIMKV_SUBMISSION_FAILED : KIMKV_RUNTIME_UNAVAILABLE;
     }
-    float time_ms[kCandidates];
-    bool usable[kCandidates];
+    float time_ms[kCandidates + 1];
+    bool usable[kCandidates + 1];
     for (int a = 0; a < n; ++a) {
         time_ms[a] = 0.0f;
         usable[a] = lt_run(st, *ctx, p, cand[a].algo, x, weights[0], y, beta, s) == HIPBLAS_STATUS_SUCCESS;
     }
+    // The kernel of few rows is one more candidate, n.
+    bool own = true;
+    for (uint32_t i = 0; i < weight_count; ++i) own = own && linear_fits(x, rows, in_features, weights[i], out_features);
+    usable[n] = own;
+    time_ms[n] = 0.0f;
+    if (own) {
+        linear_launch(x, rows, in_features, weights[0], out_features, y, y_f32 != 0, beta, s);
+        usable[n] = launch_status() == KIMKV_OK;
+    }
     for (int round = 0; round < kRounds; ++round) {
-        for (int a = 0; a < n; ++a) {
+        for (int a = 0; a <= n; ++a) {
             if (!usable[a]) continue;
             bool ok = hipEventRecord(e0, s) == hipSuccess;
             for (int i = 0; i < kReps && ok; ++i) {
                 const uint16_t* w = weights[(static_cast<uint32_t>(round * kReps + i) + static_cast<uint32_t>(a)) % weight_count];
-                ok = lt_run(st, *ctx, p, cand[a].algo, x, w, y, beta, s) == HIPBLAS_STATUS_SUCCESS;
+                if (a == n) {
+                    linear_launch(x, rows, in_features, w, out_features, y, y_f32 != 0, beta, s);
+                    ok = launch_status() == KIMKV_OK;
+                } else {
+                    ok = lt_run(st, *ctx, p, cand[a].algo, x, w, y, beta, s) == HIPBLAS_STATUS_SUCCESS;
+                }
             }
             float ms = 0.0f;
             ok = ok && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess
@@ -520,16 +724,19 @@ kimkv_status kimkv_linear_tune(const uint16_t* x, uint32_t rows, uint32_t in_fea
         }
     }
     int best = -1;
-    for (int a = 0; a < n; ++a) {
+    int library = -1;   // the best of the library's, for calls the kernel does not take
+    for (int a = 0; a <= n; ++a) {
         if (usable[a] && (best < 0 || time_ms[a] < time_ms[best])) best = a;
+        if (a < n && usable[a] && (library < 0 || time_ms[a] < time_ms[library])) library = a;
     }
     static_cast<void>(hipEventDestroy(e0));
     static_cast<void>(hipEventDestroy(e1));
-    if (best < 0) {
+    if (library < 0) {
         lt_destroy(p);
         return KIMKV_SUBMISSION_FAILED;
     }
-    p.algo = cand[best].algo;
+    p.own = best == n;
+    p.algo = cand[library].algo;
     auto it = ctx->plans.find(key);
     if (it != ctx->plans.end()) {
         lt_destroy(it->second);

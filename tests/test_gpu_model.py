@@ -179,6 +179,37 @@ def test_linear_matches_fp32_reference(dev):
     print(f"linear {rows}x{fin}x{fout}: within fp32-accumulate + fp16 rounding", flush=True)
 
 
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 32, 33, 64])
+def test_linear_few_rows(dev, rows):
+    """The kernel of few rows at the edges of its tiles: sums of one step and
+    of more steps than waves, feature counts of one tile, of a partial last
+    tile and of each tile count per workgroup (1, 300, 2056, 4104, 8200, 12296
+    features), fp16 and fp32 outputs, beta; and operands off the vectors'
+    alignment, which the library takes.  Bound: fp32 sums of up to 1088
+    products (|x w| <= 0.25 of rms 0.05 each) and one fp16 rounding."""
+    rng = np.random.default_rng(rows)
+    for fin, fout in [(64, 300), (1088, 1), (576, 2056), (64, 4104), (64, 8200), (128, 12296)]:
+        x, w = _f16(rng, (rows, fin), 1.0), _f16(rng, (fout, fin), 0.05)
+        y0 = _f16(rng, (rows, fout), 1.0)
+        prod = x.astype(np.float64) @ w.astype(np.float64).T
+        for off in (0, 1):   # halves off the 16-byte grid
+            xb = dev.upload(np.concatenate([np.zeros(off, np.float16), x.reshape(-1)]).view(np.uint16))
+            wb = dev.upload(w.view(np.uint16))
+            for y_f32, beta in ((False, 0.0), (False, 0.5), (True, 1.0)):
+                print(f"linear {rows}x{fin}x{fout} off={off} f32={y_f32} beta={beta}", flush=True)
+                y = np.concatenate([y0.reshape(-1), np.full(64, 7.0, np.float16)])
+                yb = dev.upload(y.astype(np.float32) if y_f32 else y.view(np.uint16))
+                dev.linear(xb.ptr + 2 * off, rows, fin, wb.ptr, fout, yb.ptr, y_f32, beta)
+                dev.sync()
+                got = dev.download(yb.ptr, (rows * fout + 64,), np.float32 if y_f32 else np.uint16)
+                got = (got if y_f32 else got.view(np.float16)).astype(np.float64)
+                want = prod + beta * y0.astype(np.float64)
+                rel = 1e-5 if y_f32 else 2.0 ** -10
+                err = np.abs(got[:rows * fout].reshape(rows, fout) - want)
+                assert np.all(err <= 1e-4 + rel * np.abs(want)), (fin, fout, off, y_f32, beta, float(err.max()))
+                assert np.all(got[rows * fout:] == 7.0)
+
+
 def _write_archive(directory, cfg, seed, corrupt=False):
     """The seeded runner's weights as a checkpoint archive: fp16 data file plus
     weight manifest (Hugging Face Llama tensor names, per-tensor SHA-256)."""
