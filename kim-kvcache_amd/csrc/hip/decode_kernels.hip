@@ -1265,10 +1265,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 
 // Merges the per-chunk partials of every multi-chunk lane.  Block = (lane,
 // 4 query heads), one wave per head.  Chunks are taken 64 at a time: lane k
-// reads chunk k's (m, l) and every lane reads its kDims dims of the chunks'
-// partial rows in the same round of loads, so a lane with up to 64 chunks
-// (and D <= 64) is merged after a single memory round trip; rounds of 64
-// chunks fold into the running (M, den, acc) like an online softmax.
+// reads chunk k's (m, l) and every lane reads its kDims dims of the first
+// kRows / kDims partial rows in the same round of loads, then of the next;
+// rounds of 64 chunks fold into the running (M, den, acc) like an online
+// softmax.  kRows = 16 unless the lanes have many chunks (launch_decode): the
+// unrolled rows run once, so their instructions come from memory, and 64 of
+// them cost more than the second round of loads that 17 rows take (200 lanes
+// of 100..900 tokens with the decode 41.0 -> 32.5 us, 8 lanes of up to 3000
+// 12.6 -> 10.6, 48 lanes of up to 6000 39.2 -> 37.8).
 constexpr unsigned kCombineHeads = 4;
 
 // Where the merge of a record launch finds its lanes: each lane's output
@@ -1287,14 +1291,14 @@ struct NoCombineLaneArgs {};
 // slots: when non-null, the lanes' merge records the decode launch tagged
 // `tag` replace the items and the chunk prefix.  With CombineLaneArgs the
 // launch arguments replace all three.
-template <uint32_t kDims, typename LaneArgs>
+template <uint32_t kDims, uint32_t kRows, typename LaneArgs>
 __global__ __launch_bounds__(64 * kCombineHeads) void combine_kernel(PoolView P, const kimkv_decode_item* items,
                                                                     const uint32_t* prefix, uint32_t total_chunks,
                                                                     uint32_t QH, uint32_t D, float* partials,
                                                                     const DecodeLaneSlot* slots, uint64_t tag,
                                                                     LaneArgs la)
 {
-    constexpr uint32_t kBatch = 64 / kDims;   // partial rows held in registers at once
+    constexpr uint32_t kBatch = kRows / kDims;   // partial rows held in registers at once
     uint32_t const lane = blockIdx.x;
     uint32_t const q = blockIdx.y * kCombineHeads + (threadIdx.x >> 6);
     uint32_t const l = threadIdx.x & 63u;
@@ -1534,10 +1538,20 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
         }
     } else {
         // Streamed K/V loads for long chunks (a workgroup streams at least
-        // 2048 tokens) or more than one round of resident workgroups (two
-        // per CU); cached loads for the short, latency-bound launches.
+        // 2048 tokens), more than one round of resident workgroups (two
+        // per CU), or a launch that reads much: from about 96 MB of pages
+        // on, which no cache keeps until the next pass (48 lanes of up to
+        // 6000 tokens 37.8 -> 34.4 us, 16 of up to 4000 of 8 x 128 31.8 ->
+        // 28.4).  Cached loads for the short, latency-bound launches (20
+        // lanes of up to 900 tokens 10.2, streamed 11.1; 3 of up to 20000 of
+        // 8 x 64, 89 MB, 20.0 and 20.7), and where the engine launches:
+        // its lanes may share pages, which the caches serve (32 lanes on
+        // shared prefixes, 22 layers twice: 1165 us, streamed 1245).
         uint64_t const resident = 2ull * (storage->compute_units > 0 ? storage->compute_units : 256);
-        bool const stream_loads = chunk_tokens >= 2048 || static_cast<uint64_t>(grid.x) * grid.y > resident;
+        uint64_t const page_bytes =
+            4ull * total_chunks * chunk_tokens * storage->layout.kv_heads * storage->layout.head_dim;
+        bool const stream_loads = chunk_tokens >= 2048 || static_cast<uint64_t>(grid.x) * grid.y > resident
+            || (!records && writes == nullptr && page_bytes >= (96ull << 20));
         PoolView const pv = pool_view(*storage);
         auto go = [&](auto dim, auto split, auto stream_kv, auto src) {
             constexpr uint32_t kD = decltype(dim)::value;
@@ -1585,19 +1599,22 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
         dim3 const cgrid(lane_count, (query_heads + kCombineHeads - 1) / kCombineHeads);
         uint32_t const D = storage->layout.head_dim;
         auto merge = [&](auto la) {
-            if (D <= 64) {
-                combine_kernel<1><<<cgrid, 64 * kCombineHeads, 0, s>>>(pool_view(*storage), device_items,
-                                                                         device_chunk_prefix, total_chunks,
-                                                                         query_heads, D, partials, slots, tag, la);
-            } else if (D <= 128) {
-                combine_kernel<2><<<cgrid, 64 * kCombineHeads, 0, s>>>(pool_view(*storage), device_items,
-                                                                         device_chunk_prefix, total_chunks,
-                                                                         query_heads, D, partials, slots, tag, la);
-            } else {
-                combine_kernel<4><<<cgrid, 64 * kCombineHeads, 0, s>>>(pool_view(*storage), device_items,
-                                                                         device_chunk_prefix, total_chunks,
-                                                                         query_heads, D, partials, slots, tag, la);
-            }
+            auto run = [&](auto dims, auto rows) {
+                combine_kernel<decltype(dims)::value, decltype(rows)::value><<<cgrid, 64 * kCombineHeads, 0, s>>>(
+                    pool_view(*storage), device_items, device_chunk_prefix, total_chunks, query_heads, D, partials, slots,
+                    tag, la);
+            };
+            // 64 rows at once from 32 chunks a lane on, where the rounds
+            // cost more than the instructions (one lane of 30000 tokens, 118
+            // chunks: 18.6 us, 19.5 by 16 rows).
+            bool const many = total_chunks > 32ull * lane_count;
+            auto pick = [&](auto dims) {
+                if (many) run(dims, std::integral_constant<uint32_t, 64>{});
+                else run(dims, std::integral_constant<uint32_t, 16>{});
+            };
+            if (D <= 64) pick(std::integral_constant<uint32_t, 1>{});
+            else if (D <= 128) pick(std::integral_constant<uint32_t, 2>{});
+            else pick(std::integral_constant<uint32_t, 4>{});
         };
         if (records && host_prefix != nullptr) {
             CombineLaneArgs la{};

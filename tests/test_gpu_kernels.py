@@ -907,6 +907,14 @@ def test_decode_combine_wide_heads_and_many_chunks(dev):
     assert (20000 + length - 1) // length > 64
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("lanes", [[15, 16, 17], [31, 33, 65, 1], [33, 65]])
+def test_decode_combine_round_edges(dev, lanes, dim):
+    """Merges at the edges of their rounds (16 rows at once, 64 from a mean of
+    more than 32 chunks a lane on): lanes of `lanes` chunks of 64 tokens."""
+    _decode_case(dev, (1, 2, dim), [64 * n - 5 for n in lanes], G=4, seed=31, chunk=64)
+
+
 def test_decode_full_step_counts(dev):
     # Chunks of 1..9 full 64-token steps, odd and even, with and without a tail.
     _decode_case(dev, (2, 4, 64), [128, 192, 256, 320, 389, 447, 511, 576], G=8, seed=16)
