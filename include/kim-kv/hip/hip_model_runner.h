@@ -8,7 +8,7 @@
 // decode step (one position) goes through a token transaction and the fused
 // split-K decode kernel, a prompt chunk (several positions) through a
 // PrefillChunk and the MFMA chunked-prefill kernel; the dense layers run on
-// all positions of the call at once (rocBLAS GEMMs, fused RMSNorm / RoPE /
+// all positions of the call at once (linear layers of kimkv_linear, fused RMSNorm / RoPE /
 // SwiGLU / argmax kernels).
 
 #include "kim-kv/engine/generation.h"

@@ -598,14 +598,18 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
  * src/cuda/model/runner_support.cpp:207-250.  Activations are fp16 rows,
  * stored with round-to-nearest-even; all accumulation is fp32. */
 
-/* y[rows][out] = x[rows][in] . weight[out][in]^T + beta * y (hipBLASLt, fp32
+/* y[rows][out] = x[rows][in] . weight[out][in]^T + beta * y (fp32
  * accumulate).  y is fp16 (y_f32 = 0) or fp32 (y_f32 != 0); beta = 1 with
- * y = the residual stream fuses the residual add.  Each exact problem (rows,
- * in, out, output type, beta != 0) keeps one algorithm per stream: the
- * library's first heuristic choice unless kimkv_linear_tune chose one. */
+ * y = the residual stream fuses the residual add.  Few rows (16; 32 up to
+ * 12288 features, 64 up to 4096; in a multiple of 64, x and weight 16-byte
+ * aligned) run on this library's own kernel, the rest on hipBLASLt.  Each
+ * exact problem (rows, in, out, output type, beta != 0) keeps one algorithm
+ * per stream: that rule's, with hipBLASLt's first heuristic choice, unless
+ * kimkv_linear_tune chose one. */
 kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features, const uint16_t* weight,
                           uint32_t out_features, void* y, int y_f32, float beta, kimkv_stream_t stream);
-/* Times the library's leading candidates for this exact problem (the stream
+/* Times hipBLASLt's leading candidates and, where it fits, this library's own
+ * kernel for this exact problem (the stream
  * is synchronized; y is overwritten or accumulated into several times, so
  * pass scratch contents) and makes the fastest the one kimkv_linear uses for
  * the problem on this stream.  Successive timed products cycle through the

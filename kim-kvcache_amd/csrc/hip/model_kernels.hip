@@ -372,15 +372,18 @@ __global__ __launch_bounds__(kLinearBlock) void linear_kernel(const uint16_t* x,
 }
 
 // What the kernel above takes: whole steps of 64, 16-byte vectors of x and w,
-// and few enough rows for the features.  Every workgroup reads its rows whole, so
-// the more workgroups the features make, the fewer rows pay: one tile a
-// workgroup up to 64 rows (5632 x 2048: 11.4 us, 17.3 in the library), up to
-// three up to 32 (2048 x 11264, 32 rows: 13.2 against 15.0; 60 rows 16.2
-// against 15.0 of GPU time), any number up to 16 (32000 features, 16 rows:
-// 28.8 against 32.0; 64 rows 39 against 33).
+// and few enough rows for the features.  Every workgroup reads its rows whole,
+// so the more workgroups the features make, the fewer rows pay: up to 16 rows
+// any number (32000 features, 16 rows: 28.8 us against 32.0; 64 rows 39
+// against 33), up to 32 one round of three tiles each (2048 x 11264, 32 rows:
+// 13.2 against 15.0; 60 rows 16.2 against 15.0 of GPU time), up to 64 only
+// products of 16 MB of weights, which the library's call outlasts (2048 x
+// 2048: 4.9 against 11.2; 5632 x 2048, 60 rows, is no faster than the
+// library's once the GPU and not the host is what a program waits for).
 bool linear_fits(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* w, uint32_t out)
 {
-    uint32_t const most = out <= 256 * 16 ? 64 : out <= 768 * 16 ? 32 : 16;
+    bool const small = out <= 256 * 16 && static_cast<uint64_t>(in) * out <= (8u << 20);
+    uint32_t const most = small ? 64 : out <= 768 * 16 ? 32 : 16;
     return rows <= most && in % 64 == 0
         && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;
 }
