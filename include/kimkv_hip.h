@@ -601,8 +601,8 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
 /* y[rows][out] = x[rows][in] . weight[out][in]^T + beta * y (fp32
  * accumulate).  y is fp16 (y_f32 = 0) or fp32 (y_f32 != 0); beta = 1 with
  * y = the residual stream fuses the residual add.  Few rows (16; 32 up to
- * 12288 features, 64 up to 4096; in a multiple of 64, x and weight 16-byte
- * aligned) run on this library's own kernel, the rest on hipBLASLt.  Each
+ * 12288 features, 64 up to 4096 features and 16 MB of weights; in a multiple
+ * of 64, x and weight 16-byte aligned) run on this library's own kernel, the rest on hipBLASLt.  Each
  * exact problem (rows, in, out, output type, beta != 0) keeps one algorithm
  * per stream: that rule's, with hipBLASLt's first heuristic choice, unless
  * kimkv_linear_tune chose one. */

@@ -246,9 +246,10 @@ __global__ __launch_bounds__(kBlock) void argmax_kernel(const float* logits, uin
 // operand order in LDS of its own, so no wave waits for another, and has the
 // next kDepth steps in flight.  The eight partial tiles are summed in LDS in
 // a fixed order.  Against the library's best of 16 (a call costs it 10 us of
-// host work), K x features, 1 and 64 rows: 2048 x 2048 4.6 and 4.9 us (11.4
-// and 11.2), 5632 x 2048 7.0 and 11.4 us (11.4 and 17.3); 1 row, 2048 x 11264
-// 11.8 us (15.1; 3.9 TB/s of weights), 2048 x 32000 27.1 us (32.0).
+// host work), K x features, 1 and 32 rows: 2048 x 2048 4.6 and 4.9 us (11.4
+// and 11.2), 2048 x 11264 11.8 and 13.2 us (15.1 and 15.0; 3.9 TB/s of
+// weights), 5632 x 2048 7.0 and 8.6 us (11.4 and 14.8); 2048 x 32000, 1 row,
+// 27.1 us (32.0).
 constexpr unsigned kLinearWaves = 8;
 constexpr unsigned kLinearBlock = 64 * kLinearWaves;
 
@@ -394,7 +395,7 @@ void linear_launch(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t
     // One workgroup per CU: as many feature tiles each as that takes, up to
     // four, or the rows in two blocks where that still fits (the second
     // block, on the same XCD when the tiles are a multiple of 8, reads the
-    // weights from its L2: 5632 x 2048, 64 rows, 16.8 us as one, 11.4 as two).
+    // weights from its L2: 5632 x 2048, 32 rows, 11.7 us as one, 8.6 as two).
     uint32_t const tiles = (out + 15) / 16;
     uint32_t const halves = rows > 16 && tiles <= 128 ? 2 : 1;
     uint32_t const block_rows = (rows + halves - 1) / halves;
