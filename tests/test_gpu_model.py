@@ -6,6 +6,9 @@ tests/test_model_oracle.py) with the same seeded weights: logits within
 0.035 max-abs (the reference's bar) and every greedy token the oracle's
 argmax up to that tolerance.  Generation is teacher-forced with the GPU's
 tokens so a near-tie cannot make the sequences diverge."""
+import hashlib
+import threading
+
 import numpy as np
 import pytest
 
@@ -208,6 +211,40 @@ def test_linear_few_rows(dev, rows):
                 err = np.abs(got[:rows * fout].reshape(rows, fout) - want)
                 assert np.all(err <= 1e-4 + rel * np.abs(want)), (fin, fout, off, y_f32, beta, float(err.max()))
                 assert np.all(got[rows * fout:] == 7.0)
+
+
+def test_linear_tune_chooses_alike(dev):
+    """A problem whose candidates lie a few percent apart, its weights read
+    from HBM (24 layers' matrices), on a host that is busy otherwise: every
+    tuning of it takes the same algorithm, which shows in the product's bits."""
+    rng = np.random.default_rng(5)
+    rows, n, layers = 128, 2048, 24
+    x, y0 = _f16(rng, (rows, n), 1.0).view(np.uint16), _f16(rng, (rows, n), 1.0).view(np.uint16)
+    xb, wb = dev.upload(x), dev.DeviceBuffer(2 * layers * n * n)
+    dev.fill_rows(wb.ptr, layers * n * n, 7, 0, n)
+    stop, blob = threading.Event(), bytes(1 << 22)
+
+    def busy():
+        while not stop.is_set():
+            hashlib.sha256(blob).digest()
+
+    others = [threading.Thread(target=busy) for _ in range(32)]
+    for t in others:
+        t.start()
+    try:
+        seen = set()
+        for _ in range(30):
+            yb = dev.upload(y0)
+            dev.linear_tune(xb.ptr, rows, n, [wb.ptr + 2 * i * n * n for i in range(layers)], n, yb.ptr, False, 1.0)
+            dev.copy_to_device(yb.ptr, y0)
+            dev.linear(xb.ptr, rows, n, wb.ptr, n, yb.ptr, False, 1.0)
+            dev.sync()
+            seen.add(dev.download(yb.ptr, (rows, n), np.uint16).tobytes())
+    finally:
+        stop.set()
+        for t in others:
+            t.join()
+    assert len(seen) == 1
 
 
 def _write_archive(directory, cfg, seed, corrupt=False):
