@@ -602,10 +602,12 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
  * accumulate).  y is fp16 (y_f32 = 0) or fp32 (y_f32 != 0); beta = 1 with
  * y = the residual stream fuses the residual add.  Few rows (16; 32 up to
  * 12288 features, 64 up to 4096 features and 16 MB of weights; in a multiple
- * of 64, x and weight 16-byte aligned) run on this library's own kernel, the rest on hipBLASLt.  Each
- * exact problem (rows, in, out, output type, beta != 0) keeps one algorithm
- * per stream: that rule's, with hipBLASLt's first heuristic choice, unless
- * kimkv_linear_tune chose one. */
+ * of 64, x and weight 16-byte aligned) run on this library's own kernel, the
+ * rest on hipBLASLt's first heuristic choice, kept per exact problem (rows,
+ * in, out, output type, beta != 0) and stream.  Which of the two a call takes
+ * follows from the call alone, not from earlier calls, unless
+ * kimkv_linear_tune chose for its problem: then the tuned algorithm, or the
+ * library's best where the own kernel won and the addresses are not aligned. */
 kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features, const uint16_t* weight,
                           uint32_t out_features, void* y, int y_f32, float beta, kimkv_stream_t stream);
 /* Times hipBLASLt's leading candidates and, where it fits, this library's own

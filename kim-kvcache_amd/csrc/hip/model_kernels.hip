@@ -660,6 +660,7 @@ kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features
             return KIMKV_SUBMISSION_FAILED;
         }
         p.algo = cand[0].algo;
+        p.own = true;   // untuned: a call the rule gives to the own kernel still takes it
         it = ctx->plans.emplace(key, p).first;
     }
     if (it->second.own && fits) {

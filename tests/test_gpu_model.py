@@ -213,6 +213,29 @@ def test_linear_few_rows(dev, rows):
                 assert np.all(got[rows * fout:] == 7.0)
 
 
+@pytest.mark.parametrize("tuned", [False, True])
+def test_linear_aligned_after_misaligned(dev, tuned):
+    """A call of a problem with x off the 16-byte grid (the library's) leaves
+    the aligned calls of that problem as they were, bit for bit."""
+    rng = np.random.default_rng(8)
+    rows, fin, fout = 11, 1344, 520   # sizes no other test uses: the stream has no plan for them yet
+    fin += 64 * tuned
+    x, w = _f16(rng, (rows, fin), 1.0), _f16(rng, (fout, fin), 0.05)
+    xb = [dev.upload(np.concatenate([np.zeros(off, np.float16), x.reshape(-1)]).view(np.uint16)) for off in (0, 1)]
+    wb, yb = dev.upload(w.view(np.uint16)), dev.DeviceBuffer(rows * fout * 4)
+    if tuned:
+        dev.linear_tune(xb[0].ptr, rows, fin, [wb.ptr], fout, yb.ptr, True, 0.0)
+    got = []
+    for off in (0, 1, 0, 1, 0):
+        dev.linear(xb[off].ptr + 2 * off, rows, fin, wb.ptr, fout, yb.ptr, True, 0.0)
+        dev.sync()
+        got.append(dev.download(yb.ptr, (rows, fout), np.float32))
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert all(np.abs(g - want).max() <= 1e-4 + 1e-5 * np.abs(want).max() for g in got)   # as in test_linear_few_rows
+    assert np.array_equal(got[0], got[2]) and np.array_equal(got[0], got[4])
+    assert np.array_equal(got[1], got[3])
+
+
 def test_linear_tune_chooses_alike(dev):
     """A problem whose candidates lie a few percent apart, its weights read
     from HBM (24 layers' matrices), on a host that is busy otherwise: every
