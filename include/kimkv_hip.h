@@ -601,9 +601,9 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
 /* y[rows][out] = x[rows][in] . weight[out][in]^T + beta * y (fp32
  * accumulate).  y is fp16 (y_f32 = 0) or fp32 (y_f32 != 0); beta = 1 with
  * y = the residual stream fuses the residual add.  Few rows (16; 32 up to
- * 12288 features, 64 up to 4096 features and 16 MB of weights; in a multiple
- * of 64, x and weight 16-byte aligned) run on this library's own kernel, the
- * rest on hipBLASLt's first heuristic choice, kept per exact problem (rows,
+ * 12288 features, 64 up to 4096 features of sums up to 4096 and 16 MB of
+ * weights; in a multiple of 64, x and weight 16-byte aligned) run on this
+ * library's own kernel, the rest on hipBLASLt's first heuristic choice, kept per exact problem (rows,
  * in, out, output type, beta != 0) and stream.  Which of the two a call takes
  * follows from the call alone, not from earlier calls, unless
  * kimkv_linear_tune chose for its problem: then the tuned algorithm, or the

@@ -381,10 +381,15 @@ __global__ __launch_bounds__(kLinearBlock) void linear_kernel(const uint16_t* x,
 // 13.2 against 15.0; 60 rows 16.2 against 15.0 of GPU time), up to 64 only
 // products of 16 MB of weights, which the library's call outlasts (2048 x
 // 2048: 4.9 against 11.2; 5632 x 2048, 60 rows, is no faster than the
-// library's once the GPU and not the host is what a program waits for).
+// library's once the GPU and not the host is what a program waits for), and
+// of sums up to 4096, which no workgroup spends long on: the library splits
+// longer ones over more of them (GPU time of 64 rows, untuned, 4096 x 512 6.5
+// us against 8.2, 5632 x 512 8.2 against 7.5, 65536 x 64 61 against 44).  Up
+// to 32 rows there is no such length: 1 to 4096 features of sums of 256 to
+// 65536 take 0.46 to 1.0 of the library's time.
 bool linear_fits(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* w, uint32_t out)
 {
-    bool const small = out <= 256 * 16 && static_cast<uint64_t>(in) * out <= (8u << 20);
+    bool const small = out <= 256 * 16 && in <= 4096 && static_cast<uint64_t>(in) * out <= (8u << 20);
     uint32_t const most = small ? 64 : out <= 768 * 16 ? 32 : 16;
     return rows <= most && in % 64 == 0
         && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15u) == 0;

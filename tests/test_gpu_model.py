@@ -236,6 +236,27 @@ def test_linear_aligned_after_misaligned(dev, tuned):
     assert np.array_equal(got[1], got[3])
 
 
+@pytest.mark.parametrize("rows,fin,own", [(64, 4096, True), (64, 4160, False), (33, 4160, False), (32, 4160, True)])
+def test_linear_rows_by_length_of_sum(dev, rows, fin, own):
+    """More than 32 rows take the own kernel for sums of up to 4096: past
+    that the aligned call gives the library's bits (those of x off the
+    16-byte grid)."""
+    rng = np.random.default_rng(9)
+    fout = 192
+    x, w = _f16(rng, (rows, fin), 1.0), _f16(rng, (fout, fin), 0.05)
+    wb, got = dev.upload(w.view(np.uint16)), []
+    for off in (0, 1):
+        xb = dev.upload(np.concatenate([np.zeros(off, np.float16), x.reshape(-1)]).view(np.uint16))
+        yb = dev.DeviceBuffer(rows * fout * 4)
+        dev.linear(xb.ptr + 2 * off, rows, fin, wb.ptr, fout, yb.ptr, True, 0.0)
+        dev.sync()
+        got.append(dev.download(yb.ptr, (rows, fout), np.float32))
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    # 4160 products of rms 0.05 in fp32: |sum| < 20, 65 steps of 64 each rounded to 2^-24 of it.
+    assert all(np.abs(g - want).max() <= 65 * 20 * 2.0 ** -24 * 4 for g in got)
+    assert np.array_equal(got[0], got[1]) != own
+
+
 def test_linear_tune_chooses_alike(dev):
     """A problem whose candidates lie a few percent apart, its weights read
     from HBM (24 layers' matrices), on a host that is busy otherwise: every
