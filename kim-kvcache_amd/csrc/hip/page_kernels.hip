@@ -50,11 +50,17 @@ __device__ inline uint32_t div_mod(uint32_t x, Divisor v, uint32_t* rem)
     return q;
 }
 
-// k_offset and v_offset (device_common.h) in 32 bits and without their
-// divisions: d < D and t < cap, so the column block is a shift or 0, which
-// the compiler cannot tell of a width that is 32 or the whole row.  A copy
-// computes two such offsets for 16 bytes; the attention kernels, which
-// compute few, are 4% slower with this form (a branch per operand load).
+// k_offset and v_offset (device_common.h) without their divisions: d < D and
+// t < cap, so the column block is a shift or 0, which the compiler cannot
+// tell of a width that is 32 or the whole row.  A copy computes two such
+// offsets for 16 bytes; the attention kernels, which compute few, are 4%
+// slower with this form (a branch per operand load).  In 32 bits, which hold
+// every offset of one head's block of 2 cap D elements (cap < 2^16) as long
+// as D <= kMaxDim32; in 64 bits the prompts' append and promotion are 1.5%
+// slower.  The paths that use them are closed to wider heads, which copy
+// element by element at k_offset and v_offset.
+constexpr uint32_t kMaxDim32 = 32768;
+
 __device__ inline uint32_t k_at(uint32_t cap, uint32_t D, uint32_t t, uint32_t d)
 {
     return D % 32u == 0u ? (d >> 5) * cap * 32u + t * 32u + (d & 31u) : t * D + d;
@@ -64,6 +70,9 @@ __device__ inline uint32_t v_at(uint32_t cap, uint32_t D, uint32_t t, uint32_t d
 {
     return cap * D + (cap % 32u == 0u ? (t >> 5) * D * 32u + d * 32u + (t & 31u) : d * cap + t);
 }
+
+// Whether 16-byte pieces of 8 dims take k_at and v_at.
+__device__ inline bool wide_dim(uint32_t D) { return D % 8u == 0u && D <= kMaxDim32; }
 
 // Entries of one wave's table read: lane i holds entry idx + i; token lane of
 // the tile is resolved from the entry that covers it.  Returns whether entry
@@ -170,7 +179,8 @@ struct AppendDivisors {
 // x 22 layers 57 us instead of 40).  Element by element the copy was seven
 // dependent rounds for a 7-token tail of 4 heads x 64; the append of 64 lanes
 // x 22 layers, a quarter of the tails copied, went from 12.6 to 7.7 us.
-// Both capacities and D are multiples of 8; src and dst are the layer's blocks.
+// Both capacities and D are multiples of 8; src and dst are the layer's
+// blocks, of fewer than 2^32 elements each.
 __device__ inline void copy_tokens_wide(const AppendDivisors& dv, uint32_t n, const uint16_t* src, uint32_t scap,
                                         uint16_t* dst, uint32_t dcap)
 {
@@ -216,7 +226,9 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         uint16_t const* src = page_base(P, job.cow_kind, job.cow_slot, scap);
         uint32_t const n = job.cow_tokens;
         if (src != nullptr && n <= scap && n <= dcap && n <= job.dst_token) {
-            if (((D | scap | dcap) & 7u) == 0) {
+            // The copy's offsets from the layer's blocks are 32 bits (64: the 64-lane append 0.2 us slower).
+            bool const small = ((P.micro_slot_elements | P.extent_slot_elements) >> 32) == 0;
+            if (small && ((D | scap | dcap) & 7u) == 0) {
                 copy_tokens_wide(dv, n, src + head_block(P, scap, layer, 0), scap, dst + head_block(P, dcap, layer, 0), dcap);
             } else {
                 uint32_t const per_head = n * D;
@@ -227,8 +239,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
                     uint32_t const d = rem - t * D;
                     uint64_t const sh = head_block(P, scap, layer, h);
                     uint64_t const dh = head_block(P, dcap, layer, h);
-                    dst[dh + k_at(dcap, D, t, d)] = src[sh + k_at(scap, D, t, d)];
-                    dst[dh + v_at(dcap, D, t, d)] = src[sh + v_at(scap, D, t, d)];
+                    dst[dh + k_offset(dcap, D, t, d)] = src[sh + k_offset(scap, D, t, d)];
+                    dst[dh + v_offset(dcap, D, t, d)] = src[sh + v_offset(scap, D, t, d)];
                 }
             }
         }
@@ -240,7 +252,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
     const uint16_t* sk = job.src_key + layer_off;
     const uint16_t* sv = job.src_value + layer_off;
     uint32_t const stride = job.src_token_stride;
-    bool const src_aligned = (D & 7u) == 0 && (stride & 7u) == 0
+    bool const src_aligned = wide_dim(D) && (stride & 7u) == 0
         && ((reinterpret_cast<uintptr_t>(sk) | reinterpret_cast<uintptr_t>(sv)) & 15u) == 0;
     if (src_aligned) {
         // K: 16-byte pieces of 8 dims of one token (contiguous in source and page).
@@ -291,8 +303,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         uint64_t const so = layer_off + static_cast<uint64_t>(t) * job.src_token_stride + rem;
         uint64_t const dh = head_block(P, dcap, layer, h);
         uint32_t const pt = job.dst_token + t;
-        dst[dh + k_at(dcap, D, pt, d)] = job.src_key[so];
-        dst[dh + v_at(dcap, D, pt, d)] = job.src_value[so];
+        dst[dh + k_offset(dcap, D, pt, d)] = job.src_key[so];
+        dst[dh + v_offset(dcap, D, pt, d)] = job.src_value[so];
     }
 }
 
@@ -436,7 +448,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_
         group_ok = a.page != nullptr && b.page == a.page && (a.pt & 7u) == 0 && b.pt == a.pt + (last - 8 * tid)
             && (a.cap & 7u) == 0;
     }
-    bool const fast = __syncthreads_and(group_ok) && (D & 7u) == 0;
+    bool const fast = __syncthreads_and(group_ok) && wide_dim(D);
     bool const whole = n == kTile && cols == kRows;
 
     for (uint32_t layer = l0; layer < l1; ++layer) {
@@ -460,8 +472,8 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_
             uint32_t const h = div_mod(r, dim, &d);
             uint16_t const* hb = e.page + head_block(P, e.cap, layer, h);
             uint64_t const at = static_cast<uint64_t>(t) * HD + r;
-            k_base[at] = hb[k_at(e.cap, D, e.pt, d)];
-            v_base[at] = hb[v_at(e.cap, D, e.pt, d)];
+            k_base[at] = hb[k_offset(e.cap, D, e.pt, d)];
+            v_base[at] = hb[v_offset(e.cap, D, e.pt, d)];
         }
     }
 }
@@ -505,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void promote_kernel(PoolView P, const kimkv
     uint32_t const H = P.heads;
     uint32_t const D = P.dim;
     uint32_t const tid = threadIdx.x;
-    if ((D & 7u) == 0 && mt == 8) {
+    if (wide_dim(D) && mt == 8) {
         uint32_t const dchunks = D / 8;
         // K: (h, t, dc) 16-byte chunks.
         uint32_t const kchunks = H * et * dchunks;
@@ -541,8 +553,8 @@ __global__ __launch_bounds__(kBlock) void promote_kernel(PoolView P, const kimkv
         uint32_t const st = t % mt;
         uint64_t const sh = head_block(P, mt, layer, h);
         uint64_t const dh = head_block(P, et, layer, h);
-        dst[dh + k_at(et, D, t, d)] = s[sh + k_at(mt, D, st, d)];
-        dst[dh + v_at(et, D, t, d)] = s[sh + v_at(mt, D, st, d)];
+        dst[dh + k_offset(et, D, t, d)] = s[sh + k_offset(mt, D, st, d)];
+        dst[dh + v_offset(et, D, t, d)] = s[sh + v_offset(mt, D, st, d)];
     }
 }
 
@@ -573,7 +585,7 @@ __global__ __launch_bounds__(kBlock) void fill_table_kernel(PoolView P, const ki
             if (e.page == nullptr) continue;
             uint32_t const h = r / D;
             uint32_t const d = r - h * D;
-            e.page[head_block(P, e.cap, layer, h) + k_at(e.cap, D, e.pt, d)] =
+            e.page[head_block(P, e.cap, layer, h) + k_offset(e.cap, D, e.pt, d)] =
                 synth_f16(seed, kv_row(stream_id, layer, 0, t0 + t), r);
         }
         return;
@@ -598,13 +610,13 @@ __global__ __launch_bounds__(kBlock) void fill_table_kernel(PoolView P, const ki
                 uint32_t const hi = synth_f16(seed, kv_row(stream_id, layer, 1, t0 + tb + 2 * j + 1), r);
                 w[j] = lo | (hi << 16);
             }
-            *reinterpret_cast<uint4*>(e.page + head_block(P, e.cap, layer, h) + v_at(e.cap, D, e.pt, d)) =
+            *reinterpret_cast<uint4*>(e.page + head_block(P, e.cap, layer, h) + v_offset(e.cap, D, e.pt, d)) =
                 make_uint4(w[0], w[1], w[2], w[3]);
         } else {
             for (uint32_t t = tb; t < te; ++t) {
                 TokEntry const f = tab[t];
                 if (f.page == nullptr) continue;
-                f.page[head_block(P, f.cap, layer, h) + v_at(f.cap, D, f.pt, d)] =
+                f.page[head_block(P, f.cap, layer, h) + v_offset(f.cap, D, f.pt, d)] =
                     synth_f16(seed, kv_row(stream_id, layer, 1, t0 + t), r);
             }
         }

@@ -123,6 +123,26 @@ def test_cow_counts_keep_other_tokens(dev, shape):
     assert np.array_equal(storage.gather(table, 128), pools.gather(table, 128))
 
 
+@pytest.mark.parametrize("shape", [(258, 128), (1, 33024)])
+def test_pages_past_32_bit_offsets(dev, shape):
+    """Pages of 65528 tokens x 33024 dims: the last heads' blocks, or the last
+    dims' V rows, begin more than 2^32 elements into the page.  A prompt's
+    tokens, a copied tail and the token after it land where they belong."""
+    H, D = shape
+    storage = dev.Storage(1, H, D, 1, 2, 8, 65528)
+    kv = oracle.synth_rows(8 * 2 * H * D, 55, 0, D).reshape(2, 8, H * D)
+    buf = dev.upload(kv)
+    v = buf.ptr + 2 * 8 * H * D
+    job = np.zeros(1, dtype=dev.APPEND_JOB)
+    for src_job in [(buf.ptr, v, 0, H * D, 0, 1, 8, 0, 0, 0, 0, 1, 0),                                        # tokens 0..7
+                    (buf.ptr + 2 * 7 * H * D, v + 2 * 7 * H * D, 0, H * D, 0, 1, 1, 1, 0, 5, 5, 1, 1)]:   # 5 copied, token 7 after them
+        job[0] = src_job
+        storage.append_batch(job)
+    desc = lambda slot, n: np.array([(slot, 1, 0, n, 65528, 1)], dtype=helpers.DESC)
+    assert np.array_equal(storage.gather(desc(0, 8), 8).reshape(2, 8, H * D), kv)
+    assert np.array_equal(storage.gather(desc(1, 6), 6).reshape(2, 6, H * D), kv[:, [0, 1, 2, 3, 4, 7]])
+
+
 def test_patch_descriptors(dev):
     """kimkv_patch_descriptors: whole-table writes (one longer than a
     workgroup's 256 words) and one-entry tail patches land exactly on their
