@@ -448,7 +448,10 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_
         group_ok = a.page != nullptr && b.page == a.page && (a.pt & 7u) == 0 && b.pt == a.pt + (last - 8 * tid)
             && (a.cap & 7u) == 0;
     }
-    bool const fast = __syncthreads_and(group_ok) && wide_dim(D);
+    // A tile of fewer than 64 tokens stores its rows two bytes at a time into
+    // an output off the 16-byte grid (whole tiles have always required it).
+    bool const aligned = n == kTile || (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    bool const fast = __syncthreads_and(group_ok) && wide_dim(D) && aligned;
     bool const whole = n == kTile && cols == kRows;
 
     for (uint32_t layer = l0; layer < l1; ++layer) {
@@ -462,7 +465,8 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(PoolView P, const kimkv_
             gather_kv_fast<kRows, false>(P, tab, layer, r0, n, cols, dim, k_base, v_base, stage);
             continue;
         }
-        // Element-wise path: groups across pages or off the 8-token grid, unmapped tokens, D % 8 != 0.
+        // Element-wise path: groups across pages or off the 8-token grid, unmapped tokens, outputs off the
+        // 16-byte grid, D % 8 != 0.
         for (uint32_t i = tid; i < n * cols; i += kBlock) {
             uint32_t const t = i / cols;
             uint32_t const r = r0 + i - t * cols;

@@ -102,6 +102,23 @@ def test_gather_tile_edges_bit_exact(dev, shape, layout):
         assert np.all(got[want.size:] == 0x1234)
 
 
+@pytest.mark.parametrize("T", [1, 9, 40, 63])
+def test_gather_into_unaligned_output(dev, T):
+    """A table of fewer than 64 tokens gathered to an address off the 16-byte grid (two bytes past it)."""
+    L, H, D = 2, 4, 64
+    storage = dev.Storage(L, H, D, 64, 8)
+    pools = oracle.HostPools(L, H, D, 64, 8)
+    table = helpers.hetero_table(T, helpers.SlotAllocator(64, 8, seed=T))
+    inp = _input(L, H, D, T, seed=T)
+    _populate(dev, storage, pools, table, inp)
+    out = dev.upload(np.full(inp.size + 16, 0x1234, dtype=np.uint16))
+    desc = dev.upload(table)
+    dev.check(dev.lib().kimkv_gather(storage.h, desc.ptr, len(table), T, out.ptr + 2, None), "gather")
+    got = dev.download(out.ptr, (inp.size + 16,), np.uint16)
+    assert np.array_equal(got[1:1 + inp.size], inp.reshape(-1))
+    assert got[0] == 0x1234 and np.all(got[1 + inp.size:] == 0x1234)
+
+
 @pytest.mark.parametrize("shape", [(4, 64), (1, 8), (8, 128), (3, 12)])
 def test_cow_counts_keep_other_tokens(dev, shape):
     """A copied tail of every length: the copied and the new token land, and
