@@ -28,8 +28,8 @@
 // of up to 256 tokens on contexts of up to 1500, 8 kv heads x 128, 4 query
 // heads each: 35.8 us, 4440 us on the generic path).
 // Tables that do not keep 8-token groups aligned, head dims other than 64 and
-// 128 and group sizes that do not divide 16 take a one-row-at-a-time generic
-// path.
+// 128 and group sizes that do not divide 16 take a generic path, eight rows at
+// a time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -454,34 +454,83 @@ __device__ void prefill_wave_store(PrefillWave<kDim>& w, const kimkv_prefill_ite
     }
 }
 
-// Generic path: one (new token, query head) row at a time; lanes own keys for
-// the scores and dims for the output.
-struct GenericScratch {
-    float p[64];
-    const uint16_t* head[64];
-    uint32_t cap[64];
-    uint32_t pt[64];
-};
+// Generic path: any table, any head dim up to 256, any scale and address.
+// kGenericRows (new token, query head) rows of one KV head at a time; lanes
+// own keys for the scores and dims for the output.  Bound by the latency of
+// the page reads and the instructions around them, so the rows share each:
+// a block of the MFMA shape that ends up here holds up to 8 tokens a wave
+// where one of another shape holds one (8 kv heads x 128, 4 query heads,
+// 6-token pages: 256 new tokens on 500 2.1 ms, a row at a time 20.4, and 2.6
+// in blocks of a token a wave; 32 new tokens 0.12, 0.97 and 0.12 ms).
+constexpr uint32_t kGenericRows = 8;
 
-__device__ void prefill_row_generic(const PoolView& P, const kimkv_prefill_item& item, uint32_t h, uint32_t q,
-                                    uint32_t i, uint32_t QH, GenericScratch* scratch)
+__device__ inline float read_lane(float v, uint32_t lane)
 {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), static_cast<int>(lane)));
+}
+
+// Dims [8 c, 8 c + 8) of a key's K row; `vec`: the row is 16-byte aligned and
+// its dims come in whole octets.
+__device__ inline half8_t generic_key8(const uint16_t* hb, uint32_t cap, uint32_t D, uint32_t pt, uint32_t c, bool vec)
+{
+    half8_t v = {};
+    if (vec) {
+        v = load_half8(hb + k_offset(cap, D, pt, 8 * c));
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            uint32_t const d = 8 * c + j;
+            if (d < D) v[j] = __builtin_bit_cast(_Float16, hb[k_offset(cap, D, pt, d)]);
+        }
+    }
+    return v;
+}
+
+// Rows [r0, r0 + kGenericRows) of the n rows (new token i0 + r / G, query
+// head h * G + r % G); rows past the last repeat it and are not stored.
+__device__ void prefill_rows_generic(const PoolView& P, const kimkv_prefill_item& item, uint32_t h, uint32_t G,
+                                     uint32_t i0, uint32_t r0, uint32_t n, uint32_t QH)
+{
+    constexpr uint32_t R = kGenericRows;
     uint32_t const lane = threadIdx.x & 63u;
     uint32_t const D = P.dim;
     uint32_t const layer = item.layer;
-    uint32_t const limit = item.token_count - item.new_tokens + i;   // inclusive
+    uint32_t const T0 = item.token_count - item.new_tokens;
     float const scale2 = item.attention_scale * kLog2e;
-    const uint16_t* qv = item.query + (static_cast<uint64_t>(i) * QH + q) * D;
-    float m_run = -INFINITY;
-    float l_run = 0.0f;
-    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t t0 = 0; t0 <= limit; t0 += 64) {
+    auto token = [&](uint32_t r) { return i0 + min(r0 + r, n - 1) / G; };   // sees keys up to T0 + token, inclusive
+    auto at = [&](uint32_t r) {   // the row in query and output
+        return (static_cast<uint64_t>(token(r)) * QH + h * G + min(r0 + r, n - 1) % G) * D;
+    };
+    float q[R][4];   // dims lane + 64 k
+    uint32_t limit[R];
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        limit[r] = T0 + token(r);
+        const uint16_t* const row = item.query + at(r);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            uint32_t const d = lane + 64u * k;
+            q[r][k] = d < D ? __half2float(__ushort_as_half(row[d])) : 0.0f;
+        }
+    }
+    uint32_t const last = limit[R - 1];
+    bool const vec = (D & 7u) == 0;
+    float m_run[R], l_run[R], o[R][4];
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        m_run[r] = -INFINITY;
+        l_run[r] = 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) o[r][k] = 0.0f;
+    }
+    for (uint32_t t0 = 0; t0 <= last; t0 += 64) {
         uint32_t const t = t0 + lane;
         uint32_t idx = find_descriptor_wave(item.descriptors, item.descriptor_count, t0);
         const uint16_t* hb = nullptr;
+        const uint16_t* vb = nullptr;
         uint32_t cap = 0;
         uint32_t pt = 0;
-        if (t <= limit) {
+        if (t <= last) {
             while (idx + 1 < item.descriptor_count && item.descriptors[idx + 1].logical_token_begin <= t) ++idx;
             kimkv_block_desc const e = item.descriptors[idx];
             if (t >= e.logical_token_begin && t < e.logical_token_begin + e.valid_tokens
@@ -491,53 +540,95 @@ __device__ void prefill_row_generic(const PoolView& P, const kimkv_prefill_item&
                     cap = e.page_token_capacity;
                     pt = t - e.logical_token_begin;
                     hb = page + head_block(P, cap, layer, h);
+                    vb = hb + v_offset(cap, D, pt, 0);
                 }
             }
         }
-        float s = -INFINITY;
-        if (hb != nullptr) {
-            float dot = 0.0f;
-            for (uint32_t d = 0; d < D; ++d) {
-                dot += __half2float(__ushort_as_half(qv[d])) * __half2float(__ushort_as_half(hb[k_offset(cap, D, pt, d)]));
-            }
-            s = dot * scale2;
-        }
-        float const m_new = fmaxf(m_run, wave_max(s));
-        float const alpha = m_new == -INFINITY ? 1.0f : exp2f(m_run - m_new);
-        float const p = (hb != nullptr && m_new != -INFINITY) ? exp2f(s - m_new) : 0.0f;
-        l_run = l_run * alpha + wave_sum(p);
-        m_run = m_new;
+        float s[R];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) o[k] *= alpha;
-        scratch->p[lane] = p;
-        scratch->head[lane] = hb;
-        scratch->cap[lane] = cap;
-        scratch->pt[lane] = pt;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        uint32_t const nt = min(64u, limit + 1 - t0);
-        for (uint32_t tt = 0; tt < nt; ++tt) {
-            float const pp = scratch->p[tt];
-            const uint16_t* vb = scratch->head[tt];
-            if (vb == nullptr || pp == 0.0f) continue;
-            uint32_t const vc = scratch->cap[tt];
-            uint32_t const vp = scratch->pt[tt];
+        for (uint32_t r = 0; r < R; ++r) s[r] = 0.0f;
+        // Query elements come from the lane that owns the dim, and below the
+        // weights and V rows from the lane that owns the key: registers read
+        // across the wave, which wants every lane here.
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                uint32_t const d = lane + 64u * k;
-                if (d < D) o[k] += pp * __half2float(__ushort_as_half(vb[v_offset(vc, D, vp, d)]));
+        for (uint32_t k = 0; k < 4; ++k) {
+            if (64 * k >= D) break;
+            constexpr uint32_t kOctets = 4;   // in flight together
+            for (uint32_t c = 8 * k; c < 8 * k + 8 && 8 * c < D; c += kOctets) {
+                half8_t key[kOctets] = {};
+                if (hb != nullptr) {
+#pragma unroll
+                    for (uint32_t x = 0; x < kOctets; ++x) {
+                        if (8 * (c + x) < D) key[x] = generic_key8(hb, cap, D, pt, c + x, vec);
+                    }
+                }
+#pragma unroll
+                for (uint32_t x = 0; x < kOctets; ++x) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 8; ++j) {
+                        uint32_t const from = (8 * (c + x) + j) & 63u;   // a dim past D is zero in both
+                        float const kd = static_cast<float>(key[x][j]);
+#pragma unroll
+                        for (uint32_t r = 0; r < R; ++r) s[r] += read_lane(q[r][k], from) * kd;
+                    }
+                }
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float p[R];
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            bool const seen = hb != nullptr && t <= limit[r];
+            s[r] = seen ? s[r] * scale2 : -INFINITY;
+            float const m_new = fmaxf(m_run[r], wave_max(s[r]));
+            float const alpha = m_new == -INFINITY ? 1.0f : exp2f(m_run[r] - m_new);
+            p[r] = seen && m_new != -INFINITY ? exp2f(s[r] - m_new) : 0.0f;
+            l_run[r] = l_run[r] * alpha + wave_sum(p[r]);
+            m_run[r] = m_new;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) o[r][k] *= alpha;
+        }
+        uint32_t const nt = min(64u, last + 1 - t0);
+        auto const vb_lo = static_cast<int>(reinterpret_cast<uintptr_t>(vb));
+        auto const vb_hi = static_cast<int>(reinterpret_cast<uintptr_t>(vb) >> 32);
+        auto const vb_width = static_cast<int>(v_width(cap));
+        constexpr uint32_t kKeys = 4;   // keys whose V elements are in flight together
+        for (uint32_t tt = 0; tt < nt; tt += kKeys) {
+            uint16_t v[kKeys][4];
+#pragma unroll
+            for (uint32_t y = 0; y < kKeys; ++y) {
+                // Lanes past nt hold no key: nullptr, weights 0.
+                auto const key = static_cast<int>(tt + y);
+                uint64_t const from = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(vb_hi, key))) << 32
+                    | static_cast<uint32_t>(__builtin_amdgcn_readlane(vb_lo, key));
+                auto const vw = static_cast<uint32_t>(__builtin_amdgcn_readlane(vb_width, key));
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    uint32_t const d = lane + 64u * k;
+                    v[y][k] = from != 0 && d < D
+                        ? reinterpret_cast<const uint16_t*>(from)[static_cast<uint64_t>(d) * vw] : uint16_t{0};
+                }
+            }
+#pragma unroll
+            for (uint32_t y = 0; y < kKeys; ++y) {
+#pragma unroll
+                for (uint32_t r = 0; r < R; ++r) {
+                    float const pp = read_lane(p[r], tt + y);   // 0 past the row's limit and the keys
+                    if (pp == 0.0f) continue;                   // whatever V holds there
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) o[r][k] += pp * __half2float(__ushort_as_half(v[y][k]));
+                }
+            }
+        }
     }
-    float const inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        uint32_t const d = lane + 64u * k;
-        if (d < D) item.output[(static_cast<uint64_t>(i) * QH + q) * D + d] = __half_as_ushort(__float2half_rn(o[k] * inv));
+    for (uint32_t r = 0; r < R; ++r) {
+        if (r0 + r >= n) break;
+        float const inv = l_run[r] > 0.0f ? 1.0f / l_run[r] : 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            uint32_t const d = lane + 64u * k;
+            if (d < D) item.output[at(r) + d] = __half_as_ushort(__float2half_rn(o[r][k] * inv));
+        }
     }
 }
 
@@ -555,7 +646,6 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
     __shared__ HeadGroup groups[kSegmentGroups];
     constexpr uint32_t kTileKeys = PrefillDims<kDim>::kTileKeys;
     __shared__ KvTile<kDim> tiles[2];
-    __shared__ GenericScratch scratch[kWaves];
     __shared__ uint32_t s_item;
     __shared__ uint32_t s_generic;
     __shared__ uint32_t s_holes;
@@ -685,13 +775,13 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
             return;
         }
     }
-    // Generic path: this wave's new tokens x the G query heads, one row at a time.
-    uint32_t const g0 = i_block + wave * (per_block / kWaves);
+    // Generic path: this wave's new tokens x the G query heads.
+    uint32_t const g0 = __builtin_amdgcn_readfirstlane(i_block + wave * (per_block / kWaves));
     uint32_t const g1 = min(g0 + per_block / kWaves, item.new_tokens);
-    for (uint32_t i = g0; i < g1; ++i) {
-        for (uint32_t g = 0; g < shape.G; ++g) {
-            prefill_row_generic(P, item, h, h * shape.G + g, i, QH, &scratch[wave]);
-        }
+    if (g0 >= g1) return;
+    uint32_t const rows = (g1 - g0) * shape.G;
+    for (uint32_t r0 = 0; r0 < rows; r0 += kGenericRows) {
+        prefill_rows_generic(P, item, h, shape.G, g0, r0, rows, QH);
     }
 }
 

@@ -1250,10 +1250,11 @@ def test_fill_kv_block_matches_oracle(dev):
 # ---- chunked prefill ---------------------------------------------------------------
 
 def _prefill_case(dev, shape, cases, G, micro_tokens=8, extent_tokens=64, seed=21, uniform_pages=False,
-                  q_gain=1.0):
+                  q_gain=1.0, scale=None, q_off=0, out_off=0):
     """cases: list of (T0, n): a table of T0 + n tokens whose last n are the chunk.  Every new token's
     output must match the oracle's decode of the first T0 + i + 1 tokens with that token's query.
-    q_gain scales the queries (larger scores, sharper softmax).  Returns the worst error."""
+    q_gain scales the queries (larger scores, sharper softmax); queries and outputs lie q_off and out_off
+    halves past a 16-byte boundary.  Returns the worst error."""
     L, H, D = shape
     QH = H * G
     totals = [t0 + n for t0, n in cases]
@@ -1266,7 +1267,7 @@ def _prefill_case(dev, shape, cases, G, micro_tokens=8, extent_tokens=64, seed=2
     per, prefix, total = storage.prefill_plan([n for _, n in cases], QH)
     items = np.zeros(len(cases), dtype=dev.PREFILL_ITEM)
     keep, outs, lanes = [], [], []
-    scale = 1.0 / math.sqrt(D)
+    scale = 1.0 / math.sqrt(D) if scale is None else scale
     for i, (t0, n) in enumerate(cases):
         T = t0 + n
         table = helpers.uniform_table(T, micro_tokens, alloc) if uniform_pages else helpers.hetero_table(T, alloc)
@@ -1276,9 +1277,9 @@ def _prefill_case(dev, shape, cases, G, micro_tokens=8, extent_tokens=64, seed=2
         if q_gain != 1.0:
             q = (helpers.to_f32(q) * q_gain).astype(np.float16).view(np.uint16)
         layer = (i * 5) % L
-        dbuf, qbuf = dev.upload(table), dev.upload(q)
-        obuf = dev.DeviceBuffer(n * QH * D * 2)
-        items[i] = (dbuf.ptr, len(table), T, n, layer, qbuf.ptr, obuf.ptr, scale)
+        dbuf, qbuf = dev.upload(table), dev.upload(np.concatenate([np.zeros(q_off, np.uint16), q]))
+        obuf = dev.DeviceBuffer((n * QH * D + out_off) * 2)
+        items[i] = (dbuf.ptr, len(table), T, n, layer, qbuf.ptr + 2 * q_off, obuf.ptr + 2 * out_off, scale)
         keep += [dbuf, qbuf]
         outs.append(obuf)
         lanes.append((table, t0, n, layer, q))
@@ -1287,17 +1288,17 @@ def _prefill_case(dev, shape, cases, G, micro_tokens=8, extent_tokens=64, seed=2
     # The same batch as an ordered launch (kimkv_prefill_order placement) into
     # second output buffers: the placement must not change a single bit.
     items2 = items.copy()
-    outs2 = [dev.DeviceBuffer(n * QH * D * 2) for _, n in cases]
+    outs2 = [dev.DeviceBuffer((n * QH * D + out_off) * 2) for _, n in cases]
     for i, ob in enumerate(outs2):
-        items2[i]["output"] = ob.ptr
+        items2[i]["output"] = ob.ptr + 2 * out_off
     order = dev.prefill_order(H, D, QH, storage.info().compute_units, totals, [n for _, n in cases])
     ibuf2, obuf_order = dev.upload(items2), dev.upload(order)
     storage.prefill_ordered_launch(ibuf2.ptr, len(cases), obuf_order.ptr, len(order), QH)
     dev.sync()
     worst = 0.0
     for (table, t0, n, layer, q), obuf, obuf2 in zip(lanes, outs, outs2):
-        got = dev.download(obuf.ptr, (n, QH * D), np.uint16)
-        assert np.array_equal(got, dev.download(obuf2.ptr, (n, QH * D), np.uint16)), "ordered launch differs"
+        got = dev.download(obuf.ptr + 2 * out_off, (n, QH * D), np.uint16)
+        assert np.array_equal(got, dev.download(obuf2.ptr + 2 * out_off, (n, QH * D), np.uint16)), "ordered launch differs"
         for i in range(n):
             want = pools.paged_decode(table, t0 + i + 1, layer, QH, q[i * QH * D:(i + 1) * QH * D], scale, f32=True)
             worst = max(worst, helpers.assert_attention_close(got[i], want))
@@ -1338,6 +1339,23 @@ def test_prefill_head_dim_128(dev, G):
     _prefill_case(dev, (2, 2, 128), [(0, 1), (0, 32), (31, 33), (100, 65), (7, 129), (64, 16)], G=G, seed=86)
     _prefill_case(dev, (1, 2, 128), [(4080, 40)], G=G, seed=87)
     _prefill_case(dev, (1, 2, 128), [(300, 20), (0, 48)], G=G, seed=88, q_gain=6.0)
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 16])
+@pytest.mark.parametrize("form", ["pages", "query", "output", "negative", "zero"])
+def test_prefill_head_dim_128_generic_forms(dev, form, G):
+    """What keeps the 128-dim shape off the MFMA path: 6-token pages, queries or outputs off the vectors'
+    alignment, a scale that is not positive.  Blocks of 128 / G tokens then run on the generic path, 8 rows
+    at a time: whole and partial blocks, partial tiles of 64 keys, last batches of rows that are not full."""
+    kw = {"pages": dict(micro_tokens=6, extent_tokens=48), "query": dict(q_off=1), "output": dict(out_off=2),
+          "negative": dict(scale=-0.09), "zero": dict(scale=0.0)}[form]
+    _prefill_case(dev, (2, 2, 128), [(0, 1), (61, 33), (130, 9)], G=G, seed=91, **kw)
+
+
+@pytest.mark.parametrize("shape,G", [((1, 2, 96), 5), ((1, 1, 12), 3), ((1, 2, 256), 9), ((1, 1, 20), 16), ((1, 2, 64), 8)])
+def test_prefill_generic_rows(dev, shape, G):
+    """The generic path's batches of 8 rows over odd group sizes and head dims (whole octets of dims or not)."""
+    _prefill_case(dev, shape, [(0, 3), (60, 9), (129, 4)], G=G, seed=92, micro_tokens=6, extent_tokens=48)
 
 
 def test_prefill_generic_paths(dev):
