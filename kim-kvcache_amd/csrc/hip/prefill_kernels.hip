@@ -724,7 +724,8 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
             }
             __syncthreads();
             if (s_generic != 0) break;
-            // A group no entry covers (a table with a hole) keeps every tile on the checked loads.
+            // A group no entry covers (a table with a hole) keeps every tile on the checked loads, which
+            // count its keys as zeros; at head dim 128 the generic path skips them, as the decode does.
             if (tid == 0) s_holes = 0;
             __syncthreads();
             for (uint32_t g = tid; g < ngroups; g += kBlock) {
@@ -732,6 +733,11 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
             }
             __syncthreads();
             bool const holes = s_holes != 0;
+            if (kDim == 128 && holes) {
+                if (tid == 0) s_generic = 1;
+                __syncthreads();
+                break;
+            }
             uint32_t const ntiles = (s1 - s0 + kTileKeys - 1) / kTileKeys;
             // Tile j is computed from tiles[j % 2] while tile j + 1 sits in the
             // other register set and tile j + 2's loads are issued: each tile's

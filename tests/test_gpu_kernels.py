@@ -1352,6 +1352,54 @@ def test_prefill_head_dim_128_generic_forms(dev, form, G):
     _prefill_case(dev, (2, 2, 128), [(0, 1), (61, 33), (130, 9)], G=G, seed=91, **kw)
 
 
+def _numpy_attention(q, keys, values, scale):
+    """float64 attention of one token: q [QH][D] over keys and values [T][H][D] (all of them seen)."""
+    QH, D = q.shape
+    G = QH // keys.shape[1]
+    out = np.empty((QH, D))
+    for h in range(QH):
+        s = keys[:, h // G].astype(np.float64) @ q[h].astype(np.float64) * scale
+        w = np.exp(s - s.max())
+        out[h] = w @ values[:, h // G].astype(np.float64) / w.sum()
+    return out.reshape(-1)
+
+
+def _prefill_rows(dev, storage, table, T, n, QH, q, q_off=0):
+    """One chunk of n new tokens (layer 0), whose queries lie q_off halves past a 16-byte boundary."""
+    D = storage.head_dim
+    dbuf, obuf = dev.upload(table), dev.DeviceBuffer(n * QH * D * 2)
+    qbuf = dev.upload(np.concatenate([np.zeros(q_off, np.uint16), q.reshape(-1)]))
+    items = np.zeros(1, dtype=dev.PREFILL_ITEM)
+    items[0] = (dbuf.ptr, len(table), T, n, 0, qbuf.ptr + 2 * q_off, obuf.ptr, 1.0 / math.sqrt(D))
+    _, prefix, total = storage.prefill_plan([n], QH)
+    ibuf, pbuf = dev.upload(items), dev.upload(prefix)
+    storage.prefill_launch(ibuf.ptr, pbuf.ptr, 1, total, QH)
+    dev.sync()
+    return dev.download(obuf.ptr, (n, QH * D), np.uint16)
+
+
+@pytest.mark.parametrize("missing", [[4], [10], [0, 5, 12]])
+def test_prefill_head_dim_128_gap(dev, missing):
+    """A table without some of its 8-token pages, in the context or among the new tokens: the rows skip
+    their keys."""
+    H, D, G, T, n = 2, 128, 4, 101, 30
+    storage = dev.Storage(1, H, D, 32, 4)
+    pools = oracle.HostPools(1, H, D, 32, 4)
+    table = helpers.uniform_table(T, 8, helpers.SlotAllocator(32, 4, seed=3))
+    inp = _input(1, H, D, T, seed=94)
+    _populate(dev, storage, pools, table, inp)
+    q = oracle.synth_rows(n * H * G * D, 95, 0, D).reshape(n, H * G, D)
+    keep = np.ones(T, bool)
+    for e in missing:
+        keep[8 * e:8 * e + 8] = False
+    got = _prefill_rows(dev, storage, np.delete(table, missing), T, n, H * G, q)
+    kv = helpers.to_f32(inp[0])
+    for i in range(n):
+        seen = np.nonzero(keep[:T - n + i + 1])[0]
+        want = _numpy_attention(helpers.to_f32(q[i]), kv[0, seen], kv[1, seen], 1.0 / math.sqrt(D))
+        helpers.assert_attention_close(got[i], want)
+
+
 @pytest.mark.parametrize("shape,G", [((1, 2, 96), 5), ((1, 1, 12), 3), ((1, 2, 256), 9), ((1, 1, 20), 16), ((1, 2, 64), 8)])
 def test_prefill_generic_rows(dev, shape, G):
     """The generic path's batches of 8 rows over odd group sizes and head dims (whole octets of dims or not)."""
