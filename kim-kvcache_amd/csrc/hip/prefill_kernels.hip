@@ -454,6 +454,23 @@ __device__ void prefill_wave_store(PrefillWave<kDim>& w, const kimkv_prefill_ite
     }
 }
 
+// Whether some accumulator of the wave's rows is not finite.
+template <uint32_t kDim>
+__device__ bool prefill_wave_nonfinite(PrefillWave<kDim> const& w, const kimkv_prefill_item& item, PrefillShape shape)
+{
+    float z = 0.0f;   // stays 0 unless a term is infinite or NaN
+#pragma unroll
+    for (uint32_t cb = 0; cb < kColBlocks; ++cb) {
+        if (w.i0 + cb * shape.tpw + w.r / shape.G >= item.new_tokens) continue;
+#pragma unroll
+        for (uint32_t db = 0; db <= PrefillDims<kDim>::kDb; ++db) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) z += w.acc[db][cb][i] * 0.0f;
+        }
+    }
+    return __ballot(z != 0.0f) != 0;
+}
+
 // Generic path: any table, any head dim up to 256, any scale and address.
 // kGenericRows (new token, query head) rows of one KV head at a time; lanes
 // own keys for the scores and dims for the output.  Bound by the latency of
@@ -776,7 +793,13 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_kernel(PoolView P, const ki
                 __syncthreads();
             }
         }
-        if (s_generic == 0) {
+        // A row of the MFMA path holds every key of its tile, past the row's
+        // limit too, at weight 0: times an infinite or NaN V that is NaN,
+        // where the row must not see the key.  At head dim 128 the wave's
+        // rows are then made again on the generic path, which leaves keys of
+        // weight 0 out.
+        bool const again = kDim == 128 && wave_has_rows && prefill_wave_nonfinite(w, item, shape);
+        if (s_generic == 0 && !again) {
             if (wave_has_rows) prefill_wave_store(w, item, h, shape, QH);
             return;
         }

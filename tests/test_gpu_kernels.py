@@ -1400,6 +1400,34 @@ def test_prefill_head_dim_128_gap(dev, missing):
         helpers.assert_attention_close(got[i], want)
 
 
+def test_prefill_head_dim_128_nonfinite(dev):
+    """An infinite V and a NaN K among the new tokens: earlier rows are what they are without them, and the
+    rows that see them what the generic path makes of them (the queries off the vectors' alignment)."""
+    H, D, G, T, n = 2, 128, 4, 230, 100
+    inf, nan = 0x7C00, 0x7E00
+    storage = dev.Storage(1, H, D, 32, 4)
+    pools = oracle.HostPools(1, H, D, 32, 4)
+    table = helpers.hetero_table(T, helpers.SlotAllocator(32, 4, seed=3))
+    inp = _input(1, H, D, T, seed=96)
+    inp[0, 1, 180, 0, 5] = inf
+    inp[0, 0, 215, 1, 7] = nan
+    _populate(dev, storage, pools, table, inp)
+    q = oracle.synth_rows(n * H * G * D, 97, 0, D).reshape(n, H * G, D)
+    got = _prefill_rows(dev, storage, table, T, n, H * G, q).reshape(n, H, G * D)
+    general = _prefill_rows(dev, storage, table, T, n, H * G, q, q_off=1).reshape(n, H, G * D)
+    kv = helpers.to_f32(inp[0])
+    for i in range(n):
+        t = T - n + i
+        want = _numpy_attention(helpers.to_f32(q[i]), kv[0, :t + 1], kv[1, :t + 1], 1.0 / math.sqrt(D)).reshape(H, -1)
+        for h, first in ((0, 180), (1, 215)):
+            if t < first:
+                assert np.all(np.isfinite(got[i, h].view(np.float16))), (i, h)
+                helpers.assert_attention_close(got[i, h], want[h])
+            else:
+                assert np.array_equal(got[i, h], general[i, h]), (i, h)
+                assert not np.all(np.isfinite(got[i, h].view(np.float16)))
+
+
 @pytest.mark.parametrize("shape,G", [((1, 2, 96), 5), ((1, 1, 12), 3), ((1, 2, 256), 9), ((1, 1, 20), 16), ((1, 2, 64), 8)])
 def test_prefill_generic_rows(dev, shape, G):
     """The generic path's batches of 8 rows over odd group sizes and head dims (whole octets of dims or not)."""
