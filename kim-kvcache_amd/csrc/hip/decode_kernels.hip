@@ -452,105 +452,122 @@ __device__ inline JobView job_view(const PoolView& P, const kimkv_append_job& jo
     return v;
 }
 
+// Tokens [c0, c1) for query head q of kv head h: lane i holds o[k] of dim
+// i + 64 k, every lane the running max and denominator.
+struct HeadPartial {
+    float o[4];
+    float m;
+    float l;
+};
+
+__device__ HeadPartial decode_head_generic(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t q,
+                                           uint32_t c0, uint32_t c1, WaveTokens* tokens, JobView const& jv)
+{
+    uint32_t const lane = threadIdx.x & 63u;
+    uint32_t const D = P.dim;
+    uint32_t const layer = item.layer;
+    float const scale2 = item.attention_scale * kLog2e;
+    const uint16_t* qv = item.query + static_cast<uint64_t>(q) * D;
+    float m_run = -INFINITY;
+    float l_run = 0.0f;
+    float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t t0 = c0; t0 < c1; t0 += 64) {
+        uint32_t const t = t0 + lane;
+        bool const valid = t < c1;
+        uint32_t idx = find_descriptor_wave(item.descriptors, item.descriptor_count, t0);
+        const uint16_t* page = nullptr;
+        uint32_t cap = 0;
+        uint32_t pt = 0;
+        if (valid) {
+            while (idx + 1 < item.descriptor_count
+                   && item.descriptors[idx + 1].logical_token_begin <= t) {
+                ++idx;
+            }
+            kimkv_block_desc const e = item.descriptors[idx];
+            if (t >= e.logical_token_begin && t < e.logical_token_begin + e.valid_tokens
+                && e.valid_tokens <= e.page_token_capacity) {
+                page = page_base(P, e.kind, e.slot, e.page_token_capacity);
+                cap = e.page_token_capacity;
+                pt = t - e.logical_token_begin;
+            }
+        }
+        float s = -INFINITY;
+        const uint16_t* hb = nullptr;
+        if (page != nullptr) {
+            hb = page + head_block(P, cap, layer, h);
+            const uint16_t* krow = nullptr;   // contiguous K row when the job supplies the token
+            if (jv.active && page == page_base(P, jv.dst_kind, jv.dst_slot, pool_tokens(P, jv.dst_kind))) {
+                if (pt == jv.dst_token) {
+                    krow = jv.key + static_cast<uint64_t>(h) * D;
+                    hb = jv.value + static_cast<uint64_t>(h) * D;
+                    cap = 0;
+                } else if (pt < jv.cow_tokens) {
+                    hb = page_base(P, jv.cow_kind, jv.cow_slot, jv.cow_cap) + head_block(P, jv.cow_cap, layer, h);
+                    cap = jv.cow_cap;
+                }
+            }
+            float dot = 0.0f;
+            for (uint32_t d = 0; d < D; ++d) {
+                uint16_t const kc = krow != nullptr ? krow[d] : hb[k_offset(cap, D, pt, d)];
+                dot += __half2float(__ushort_as_half(qv[d])) * __half2float(__ushort_as_half(kc));
+            }
+            s = dot * scale2;
+        }
+        float const m_new = fmaxf(m_run, wave_max(s));
+        float const alpha = m_new == -INFINITY ? 1.0f : exp2f(m_run - m_new);
+        // Same weight shift as the fast path: partials of one lane may
+        // come from both paths and are merged as they are.
+        float const p = (page != nullptr && m_new != -INFINITY) ? exp2f(s - m_new + kWeightShift) : 0.0f;
+        l_run = l_run * alpha + wave_sum(p);
+        m_run = m_new;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] *= alpha;
+        tokens->p[lane] = p;
+        tokens->head[lane] = hb;
+        tokens->cap[lane] = cap;
+        tokens->pt[lane] = pt;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint32_t const nt = min(64u, c1 - t0);
+        for (uint32_t tt = 0; tt < nt; ++tt) {
+            float const pp = tokens->p[tt];
+            const uint16_t* vb = tokens->head[tt];
+            uint32_t const vc = tokens->cap[tt];
+            uint32_t const vp = tokens->pt[tt];
+            if (vb == nullptr || pp == 0.0f) continue;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t const d = lane + 64u * k;
+                if (d < D) {
+                    uint16_t const vv = vc == 0 ? vb[d] : vb[v_offset(vc, D, vp, d)];
+                    o[k] += pp * __half2float(__ushort_as_half(vv));
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    return HeadPartial{{o[0], o[1], o[2], o[3]}, m_run, l_run};
+}
+
 __device__ void decode_wave_generic(const PoolView& P, const kimkv_decode_item& item, uint32_t h,
                                     uint32_t G, uint32_t QH, uint32_t c0, uint32_t c1,
                                     uint32_t chunk_index, bool single_chunk, WaveTokens* tokens, JobView const& jv)
 {
     uint32_t const lane = threadIdx.x & 63u;
     uint32_t const D = P.dim;
-    uint32_t const layer = item.layer;
-    float const scale2 = item.attention_scale * kLog2e;
     for (uint32_t j = 0; j < G; ++j) {
         uint32_t const q = h * G + j;
-        const uint16_t* qv = item.query + static_cast<uint64_t>(q) * D;
-        float m_run = -INFINITY;
-        float l_run = 0.0f;
-        float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (uint32_t t0 = c0; t0 < c1; t0 += 64) {
-            uint32_t const t = t0 + lane;
-            bool const valid = t < c1;
-            uint32_t idx = find_descriptor_wave(item.descriptors, item.descriptor_count, t0);
-            const uint16_t* page = nullptr;
-            uint32_t cap = 0;
-            uint32_t pt = 0;
-            if (valid) {
-                while (idx + 1 < item.descriptor_count
-                       && item.descriptors[idx + 1].logical_token_begin <= t) {
-                    ++idx;
-                }
-                kimkv_block_desc const e = item.descriptors[idx];
-                if (t >= e.logical_token_begin && t < e.logical_token_begin + e.valid_tokens
-                    && e.valid_tokens <= e.page_token_capacity) {
-                    page = page_base(P, e.kind, e.slot, e.page_token_capacity);
-                    cap = e.page_token_capacity;
-                    pt = t - e.logical_token_begin;
-                }
-            }
-            float s = -INFINITY;
-            const uint16_t* hb = nullptr;
-            if (page != nullptr) {
-                hb = page + head_block(P, cap, layer, h);
-                const uint16_t* krow = nullptr;   // contiguous K row when the job supplies the token
-                if (jv.active && page == page_base(P, jv.dst_kind, jv.dst_slot, pool_tokens(P, jv.dst_kind))) {
-                    if (pt == jv.dst_token) {
-                        krow = jv.key + static_cast<uint64_t>(h) * D;
-                        hb = jv.value + static_cast<uint64_t>(h) * D;
-                        cap = 0;
-                    } else if (pt < jv.cow_tokens) {
-                        hb = page_base(P, jv.cow_kind, jv.cow_slot, jv.cow_cap) + head_block(P, jv.cow_cap, layer, h);
-                        cap = jv.cow_cap;
-                    }
-                }
-                float dot = 0.0f;
-                for (uint32_t d = 0; d < D; ++d) {
-                    uint16_t const kc = krow != nullptr ? krow[d] : hb[k_offset(cap, D, pt, d)];
-                    dot += __half2float(__ushort_as_half(qv[d])) * __half2float(__ushort_as_half(kc));
-                }
-                s = dot * scale2;
-            }
-            float const m_new = fmaxf(m_run, wave_max(s));
-            float const alpha = m_new == -INFINITY ? 1.0f : exp2f(m_run - m_new);
-            // Same weight shift as the fast path: partials of one lane may
-            // come from both paths and are merged as they are.
-            float const p = (page != nullptr && m_new != -INFINITY) ? exp2f(s - m_new + kWeightShift) : 0.0f;
-            l_run = l_run * alpha + wave_sum(p);
-            m_run = m_new;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] *= alpha;
-            tokens->p[lane] = p;
-            tokens->head[lane] = hb;
-            tokens->cap[lane] = cap;
-            tokens->pt[lane] = pt;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            uint32_t const nt = min(64u, c1 - t0);
-            for (uint32_t tt = 0; tt < nt; ++tt) {
-                float const pp = tokens->p[tt];
-                const uint16_t* vb = tokens->head[tt];
-                uint32_t const vc = tokens->cap[tt];
-                uint32_t const vp = tokens->pt[tt];
-                if (vb == nullptr || pp == 0.0f) continue;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    uint32_t const d = lane + 64u * k;
-                    if (d < D) {
-                        uint16_t const vv = vc == 0 ? vb[d] : vb[v_offset(vc, D, vp, d)];
-                        o[k] += pp * __half2float(__ushort_as_half(vv));
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
+        HeadPartial const s = decode_head_generic(P, item, h, q, c0, c1, tokens, jv);
         if (single_chunk) {
-            float const inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+            float const inv = s.l > 0.0f ? 1.0f / s.l : 0.0f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint32_t const d = lane + 64u * k;
                 if (d < D) {
-                    item.output[static_cast<uint64_t>(q) * D + d] = __half_as_ushort(__float2half_rn(o[k] * inv));
+                    item.output[static_cast<uint64_t>(q) * D + d] = __half_as_ushort(__float2half_rn(s.o[k] * inv));
                 }
             }
         } else {
@@ -558,11 +575,11 @@ __device__ void decode_wave_generic(const PoolView& P, const kimkv_decode_item& 
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint32_t const d = lane + 64u * k;
-                if (d < D) ws[d] = o[k];
+                if (d < D) ws[d] = s.o[k];
             }
             if (lane == 0) {
-                ws[D] = m_run;
-                ws[D + 1] = l_run;
+                ws[D] = s.m;
+                ws[D + 1] = s.l;
             }
         }
     }
@@ -770,6 +787,63 @@ __device__ inline NewTokenRows new_token_rows(const DecodeLds& lds, JobView cons
     return NewTokenRows{jv.key + static_cast<uint64_t>(h) * D, jv.value + static_cast<uint64_t>(h) * D, T - 1};
 }
 
+// The same by the generic path, a query head at a time (plans choose a chunk
+// four times as long for a workgroup of one kv head, before any table is
+// seen: with one wave at work 4 lanes of 1000 tokens in 6-token pages, 8 kv
+// heads x 128, 4 query heads each, took 3.46 ms, with four 0.95).
+__device__ void decode_head_split_generic(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t G,
+                                          uint32_t QH, uint32_t s0, uint32_t s1, uint32_t chunk_index, bool single,
+                                          DecodeLds& lds, JobView const& jv)
+{
+    constexpr uint32_t kRow = 260;   // o (up to 256), m, l, pad
+    uint32_t const tid = threadIdx.x;
+    uint32_t const wave = tid >> 6;
+    uint32_t const lane = tid & 63u;
+    uint32_t const D = P.dim;
+    float* const part = reinterpret_cast<float*>(lds.groups);
+    __syncthreads();   // the table's last readers (a launch that stores it)
+    for (uint32_t j = 0; j < G; ++j) {
+        uint32_t const q = h * G + j;
+        HeadPartial s{{0.0f, 0.0f, 0.0f, 0.0f}, -INFINITY, 0.0f};
+        if (s0 < s1) s = decode_head_generic(P, item, h, q, s0, s1, &lds.wave_tokens[wave], jv);
+        float* const row = part + wave * kRow;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) row[lane + 64 * k] = s.o[k];   // zeros past D
+        if (lane == 0) {
+            row[256] = s.m;
+            row[257] = s.l;
+        }
+        __syncthreads();
+        if (tid < D) {
+            float M = -INFINITY;
+#pragma unroll
+            for (uint32_t v = 0; v < kHeadsPerBlock; ++v) M = fmaxf(M, part[v * kRow + 256]);
+            float den = 0.0f;
+            float o = 0.0f;
+#pragma unroll
+            for (uint32_t v = 0; v < kHeadsPerBlock; ++v) {
+                float const m = part[v * kRow + 256];
+                float const c = m == -INFINITY ? 0.0f : exp2f(m - M);
+                if (c == 0.0f) continue;   // whatever V made of it, as for a key of weight 0
+                den += c * part[v * kRow + 257];
+                o += c * part[v * kRow + tid];
+            }
+            if (single) {
+                float const inv = den > 0.0f ? 1.0f / den : 0.0f;
+                item.output[static_cast<uint64_t>(q) * D + tid] = __half_as_ushort(__float2half_rn(o * inv));
+            } else {
+                float* const ws = item.workspace + (static_cast<uint64_t>(chunk_index) * QH + q) * (D + 2);
+                ws[tid] = o;
+                if (tid == 0) {
+                    ws[D] = M;
+                    ws[D + 1] = den;
+                }
+            }
+        }
+        __syncthreads();   // the rows are written anew for the next head
+    }
+}
+
 template <uint32_t kDim, bool kStream>
 __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t QH,
                                         uint32_t c0, uint32_t c1, uint32_t chunk_index, bool single, bool fast,
@@ -778,15 +852,13 @@ __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_it
     uint32_t const tid = threadIdx.x;
     uint32_t const wave = tid >> 6;
     uint32_t const G = QH / P.heads;
-    if (!fast) {
-        if (wave == 0) {
-            decode_wave_generic(P, item, h, G, QH, c0, c1, chunk_index, single, &lds.wave_tokens[0], jv);
-        }
-        return;
-    }
     uint32_t const quarter = ((c1 - c0 + 3) / 4 + 63) / 64 * 64;
     uint32_t const s0 = min(c0 + wave * quarter, c1);
     uint32_t const s1 = min(s0 + quarter, c1);
+    if (!fast) {
+        decode_head_split_generic(P, item, h, G, QH, s0, s1, chunk_index, single, lds, jv);
+        return;
+    }
     WavePartial<kDim> w;
     if (s0 < s1) {
         w = decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, s0, s1,

@@ -516,7 +516,8 @@ def test_decode_lane_records_table_cache_head_split_many_rounds(dev):
 @pytest.mark.parametrize("mode,order,heads,dim", [("four_heads", 1, 4, 64), ("head_split", 1, 4, 64),
                                                   ("four_heads", -1, 4, 64), ("head_split", -1, 4, 64),
                                                   ("four_heads", 1, 8, 64), ("head_split", 1, 8, 64),
-                                                  ("four_heads", 1, 4, 128)])
+                                                  ("four_heads", 1, 4, 128), ("head_split", 1, 4, 128),
+                                                  ("four_heads", 1, 4, 96), ("head_split", 1, 4, 96)])
 def test_decode_lane_records_match_item_launch(dev, mode, order, heads, dim):
     """kimkv_paged_decode_lanes (each lane's item and job built in the kernel from a device lane record
     and the layer's evenly spaced addresses) equals kimkv_paged_decode_write_batch_slots_prefix with the
@@ -525,8 +526,8 @@ def test_decode_lane_records_match_item_launch(dev, mode, order, heads, dim):
     strides).  With a chunk table cache: the first launch of a tag builds and stores the tables, the next
     two read them, and a new tag over the same cache rebuilds them; every launch gives the same outputs.
     Malformed launches are refused without running.  With 8 kv heads a chunk has two workgroups of four
-    heads each (or eight in the head-split mode) sharing its cached table; head_dim 128 takes the
-    merge of two dims per lane."""
+    heads each (or eight in the head-split mode) sharing its cached table; head dims 128 and
+    96 (the generic path) take the merge of two dims per lane."""
     shape = (3, heads, dim)
     L, H, D = shape
     QH, layer = 32, 1
@@ -1009,6 +1010,18 @@ def test_decode_guided_slices(dev):
                  uniform_pages=True, chunk=GU)
     # 70 launches on one storage: its 64 counter slots are reused after their reset.
     _decode_case(dev, (1, 4, 64), [300, 1000, 2500], G=8, seed=66, chunk=GU, repeat=70)
+
+
+@pytest.mark.parametrize("shape,G,pages", [((1, 2, 128), 4, 6), ((1, 2, 128), 1, 6), ((1, 2, 96), 4, 8), ((1, 2, 96), 20, 8),
+                                           ((1, 1, 256), 3, 8), ((1, 3, 12), 2, 8)])
+@pytest.mark.parametrize("mode", ["head_split", "short", "four_heads", "plan", "guided"])
+def test_decode_generic_forms(dev, mode, shape, G, pages):
+    """The generic path in every mode: a chunk of one kv head cut into the four waves' quarters (all of them,
+    some, or one at work), guided lanes of one to six slices, some of them empty."""
+    chunk = {"head_split": 320 | dev.DECODE_HEAD_SPLIT, "short": 64 | dev.DECODE_HEAD_SPLIT, "four_heads": 256,
+             "plan": None, "guided": dev.DECODE_GUIDED | 64}[mode]
+    _decode_case(dev, shape, [1, 5, 63, 64, 66, 100, 131, 300, 396, 397, 1500], G=G, seed=93, chunk=chunk,
+                 micro_tokens=pages, extent_tokens=8 * pages)
 
 
 def test_decode_long_chunks(dev):
