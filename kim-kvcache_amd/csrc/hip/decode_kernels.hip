@@ -350,6 +350,22 @@ __device__ WavePartial<kDim> decode_wave_fast(const GroupEntry* groups, const Gr
     return out;
 }
 
+// Whether some accumulator of the wave's query columns is not finite.  The
+// matrix cores multiply every key's V, also at a weight that is 0 in both fp16
+// parts: times an infinite or NaN V that is NaN, where the generic path leaves
+// a key of weight 0 out and keeps an infinity.  Head dim 128 then takes that
+// path for the chunk (head dim 64 never has).
+template <uint32_t kDim>
+__device__ inline bool wave_nonfinite(WavePartial<kDim> const& w, uint32_t G)
+{
+    if (kDim != 128) return false;
+    // Stays 0 unless a term is infinite or NaN; four sums, as one is a chain of 33 dependent operations.
+    float4_t z = {w.l * 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (uint32_t db = 0; db < kDim / 16; ++db) z += w.acc[db] * 0.0f;
+    return __ballot((threadIdx.x & 15u) < G && (z[0] + z[1]) + (z[2] + z[3]) != 0.0f) != 0;
+}
+
 // Writes dims [d0, d0 + 4) of query head q: the fp16 output when the lane
 // has one chunk, else the chunk's (o, m, l) partial for combine_kernel (m and
 // l by the one caller per row that passes write_ml).
@@ -844,36 +860,18 @@ __device__ void decode_head_split_generic(const PoolView& P, const kimkv_decode_
     }
 }
 
-template <uint32_t kDim, bool kStream>
-__device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t QH,
-                                        uint32_t c0, uint32_t c1, uint32_t chunk_index, bool single, bool fast,
-                                        DecodeLds& lds, JobView const& jv)
+// The four waves' fast-path states merged in the group table's LDS, [wave]
+// [query column][kDim + 4 floats: o(kDim), m, l, pad].  Returns 0, or NaN
+// when one of the thread's merged values is not finite (as it is when one of
+// the states' values is not).
+template <uint32_t kDim>
+__device__ inline float merge_head_split(const kimkv_decode_item& item, uint32_t h, uint32_t G, uint32_t QH,
+                                        WavePartial<kDim> const& w, uint32_t chunk_index, bool single, DecodeLds& lds)
 {
     uint32_t const tid = threadIdx.x;
     uint32_t const wave = tid >> 6;
-    uint32_t const G = QH / P.heads;
-    uint32_t const quarter = ((c1 - c0 + 3) / 4 + 63) / 64 * 64;
-    uint32_t const s0 = min(c0 + wave * quarter, c1);
-    uint32_t const s1 = min(s0 + quarter, c1);
-    if (!fast) {
-        decode_head_split_generic(P, item, h, G, QH, s0, s1, chunk_index, single, lds, jv);
-        return;
-    }
-    WavePartial<kDim> w;
-    if (s0 < s1) {
-        w = decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, s0, s1,
-                                            new_token_rows(lds, jv, item.token_count, h, kDim));
-    } else {
-#pragma unroll
-        for (uint32_t db = 0; db < kDim / 16; ++db) w.acc[db] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        w.m = -INFINITY;
-        w.l = 0.0f;
-    }
-    // Every wave is done with the group table: its LDS holds the four states,
-    // [wave][query column][kDim + 4 floats: o(kDim), m, l, pad].
     constexpr uint32_t kRow = kDim + 4;
     static_assert(4 * 16 * kRow * sizeof(float) <= sizeof(lds.groups), "the states fit the group table's space");
-    __syncthreads();
     float* part = reinterpret_cast<float*>(lds.groups);
     {
         uint32_t const l = tid & 63u;
@@ -890,7 +888,8 @@ __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_it
     __syncthreads();
     // Thread t merges dims [4 (t % 16) + 64 j, +4) of query column t / 16.
     uint32_t const r = tid >> 4;
-    if (r >= G) return;
+    if (r >= G) return 0.0f;
+    float4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
     float M = -INFINITY;
 #pragma unroll
     for (uint32_t v = 0; v < kHeadsPerBlock; ++v) M = fmaxf(M, part[(v * 16 + r) * kRow + kDim]);
@@ -908,7 +907,45 @@ __device__ void decode_head_split_chunk(const PoolView& P, const kimkv_decode_it
             o += c * *reinterpret_cast<const float4_t*>(row + d0);
         }
         store_partial<kDim>(item, QH, h * G + r, chunk_index, single, o, d0, M, den, d0 == 0);
+        z += o * 0.0f;
+        z[0] += den * 0.0f;
     }
+    return (z[0] + z[1]) + (z[2] + z[3]);
+}
+
+// Returns whether the fast path's result is not finite (head dim 128, see
+// wave_nonfinite): then the caller runs the chunk again without `fast`, over
+// what was written.
+template <uint32_t kDim, bool kStream>
+__device__ bool decode_head_split_chunk(const PoolView& P, const kimkv_decode_item& item, uint32_t h, uint32_t QH,
+                                        uint32_t c0, uint32_t c1, uint32_t chunk_index, bool single, bool fast,
+                                        DecodeLds& lds, JobView const& jv)
+{
+    uint32_t const wave = threadIdx.x >> 6;
+    uint32_t const G = QH / P.heads;
+    uint32_t const quarter = ((c1 - c0 + 3) / 4 + 63) / 64 * 64;
+    uint32_t const s0 = min(c0 + wave * quarter, c1);
+    uint32_t const s1 = min(s0 + quarter, c1);
+    if (!fast) {
+        decode_head_split_generic(P, item, h, G, QH, s0, s1, chunk_index, single, lds, jv);
+        return false;
+    }
+    WavePartial<kDim> w;
+    if (s0 < s1) {
+        w = decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, s0, s1,
+                                            new_token_rows(lds, jv, item.token_count, h, kDim));
+    } else {
+#pragma unroll
+        for (uint32_t db = 0; db < kDim / 16; ++db) w.acc[db] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        w.m = -INFINITY;
+        w.l = 0.0f;
+    }
+    __syncthreads();   // every wave is done with the group table
+    float const z = merge_head_split(item, h, G, QH, w, chunk_index, single, lds);
+    if (kDim != 128) return false;
+    bool const again = __syncthreads_or(z != 0.0f) != 0;
+    if (again) __threadfence();
+    return again;
 }
 
 // Stores the lane's new token for kv heads [h0, h1) of `layer` (a job that
@@ -1218,9 +1255,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     uint32_t const wave = tid >> 6;
     if (!kSplit) {
         uint32_t const h = blockIdx.y * kHeadsPerBlock + wave;
-        if (h < H && !fast) {
-            decode_wave_generic(P, item, h, G, QH, c0, c1, chunk_index, single, &lds.wave_tokens[wave], jv);
-        } else if (h < H) {
+        bool generic = !fast;
+        if (h < H && fast) {
             WavePartial<kDim> const w =
                 decode_wave_fast<kDim, kStream>(lds.groups, GroupResolver(P, item.layer, h), item, h, G, c0, c0, c1,
                                                 new_token_rows(lds, jv, T, h, kDim));
@@ -1233,9 +1269,23 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
                                         w.m, w.l, db == 0 && l < 16);
                 }
             }
+            // Looked at behind the stores, which then wait for nothing; the generic path's follow them.
+            generic = wave_nonfinite(w, G);
+            if (generic) __threadfence();
+        }
+        if (h < H && generic) {
+            decode_wave_generic(P, item, h, G, QH, c0, c1, chunk_index, single, &lds.wave_tokens[wave],
+                                job_view(P, lds.job, jv.active));
         }
     } else if (blockIdx.y < H) {
-        decode_head_split_chunk<kDim, kStream>(P, item, blockIdx.y, QH, c0, c1, chunk_index, single, fast, lds, jv);
+        bool const again = decode_head_split_chunk<kDim, kStream>(P, item, blockIdx.y, QH, c0, c1, chunk_index, single,
+                                                                  fast, lds, jv);
+        if (kDim == 128 && again) {
+            // (The job view is made anew rather than kept in registers across the streaming loop.)
+            static_cast<void>(decode_head_split_chunk<kDim, kStream>(P, item, blockIdx.y, QH, c0, c1, chunk_index,
+                                                                     single, false, lds,
+                                                                     job_view(P, lds.job, job_ok)));
+        }
     }
     // The job comes back from LDS rather than staying in registers across
     // the streaming loop.
@@ -1283,10 +1333,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     uint32_t const G = QH / H;
     uint32_t const pairs = lane_count * H;
     uint32_t const total = pairs * K;
+    bool again = false;   // the unit's fast path was not finite: it runs once more without it
     for (;;) {
-        if (tid == 0) s_unit = atomicAdd(&counter[0], 1u);
+        if (tid == 0 && !again) s_unit = atomicAdd(&counter[0], 1u);
         __syncthreads();
-        uint32_t const u = s_unit;
+        uint32_t const u = __builtin_amdgcn_readfirstlane(s_unit);   // scalar, and with it the item and the job
         __syncthreads();   // every thread has the unit before thread 0 fetches the next
         if (u >= total) break;
         uint32_t const k = u / pairs;
@@ -1320,8 +1371,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
             for (uint32_t i = tid; i < G * (D + 2); i += kBlock) ws[i] = i % (D + 2) == D ? -INFINITY : 0.0f;
             continue;
         }
-        bool const fast = build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv);
-        decode_head_split_chunk<kDim, true>(P, item, h, QH, c0, c1, k, n == 1, fast, lds, jv);
+        bool const fast = build_chunk_table<kDim>(P, item, QH, c0, c1, lds, jv) && !again;
+        again = decode_head_split_chunk<kDim, true>(P, item, h, QH, c0, c1, k, n == 1, fast, lds, jv);
+        if (again) continue;
         // The last slice (never empty) stores the job's positions of head h.
         if (writer && job_ok) write_token_heads(P, lds.job, item.layer, h, h + 1);
         __syncthreads();   // the next unit rebuilds the table in the same LDS

@@ -1413,6 +1413,47 @@ def test_prefill_head_dim_128_gap(dev, missing):
         helpers.assert_attention_close(got[i], want)
 
 
+@pytest.mark.parametrize("mode", ["four_heads", "head_split", "split_k", "guided"])
+def test_decode_head_dim_128_nonfinite(dev, mode):
+    """Infinite and NaN values at head dim 128, as where each weight is one fp32 number: a key of weight 0
+    (its score 300 below the others') adds nothing whatever its V, an infinite V of any other weight gives
+    infinity (one of 2^-86, which fp16's parts of a weight do not hold, among them), a NaN K or V NaN."""
+    H, D, G = 2, 128, 4
+    QH = H * G
+    chunk = {"four_heads": 256, "head_split": 256 | dev.DECODE_HEAD_SPLIT, "split_k": 64,
+             "guided": dev.DECODE_GUIDED | 64}[mode]
+    storage = dev.Storage(1, H, D, 256, 32)
+    pools = oracle.HostPools(1, H, D, 256, 32)
+    alloc = helpers.SlotAllocator(256, 32, seed=3)
+    inf, nan, T = 0x7C00, 0x7E00, 64
+    q = oracle.synth_rows(QH * D, 98, 0, D)
+    q[::D] = np.float16(60.0).view(np.uint16)
+    lanes, keep, wants = [], [], []
+    # component, token, kv head, value, the key's dim 0 (times the query's 60 its score; None: the others' 0)
+    for i, (c, t, h, value, k0) in enumerate([(1, 20, 0, inf, -5.0), (1, 0, 1, nan, -5.0), (1, 63, 1, inf, -5.0),
+                                              (1, 20, 0, inf, None), (1, 41, 1, inf, -1.0), (1, 33, 1, nan, None),
+                                              (0, 40, 1, nan, None)]):
+        inp = _input(1, H, D, T, seed=990 + i)
+        inp[0, 0, :, :, 0] = 0
+        if k0 is not None:
+            inp[0, 0, t, h] = 0
+            inp[0, 0, t, h, 0] = np.float16(k0).view(np.uint16)
+        inp[0, c, t, h, 9] = value
+        table = helpers.hetero_table(T, alloc)
+        keep.append(_populate(dev, storage, pools, table, inp))
+        lanes.append((table, T, 0, q, 1.0))
+        kv = helpers.to_f32(inp[0])
+        v = np.where(np.isfinite(kv[1]), kv[1], 0.0) if k0 == -5.0 else kv[1]
+        with np.errstate(all="ignore"):
+            wants.append(_numpy_attention(helpers.to_f32(q).reshape(QH, D), kv[0], v, 1.0))
+    outs, _, _ = _run_decode(dev, storage, lanes, QH, chunk=chunk)
+    for i, (got, want) in enumerate(zip(outs, wants)):
+        value, ok = got.view(np.float16), np.isfinite(want)
+        assert np.array_equal(np.isnan(value), np.isnan(want)), (mode, i)
+        assert np.array_equal(np.isinf(value), np.isinf(want)), (mode, i)
+        assert np.all(np.abs(value[ok].astype(np.float64) - want[ok]) <= 2e-3 + 1e-3 * np.abs(want[ok])), (mode, i)
+
+
 def test_prefill_head_dim_128_nonfinite(dev):
     """An infinite V and a NaN K among the new tokens: earlier rows are what they are without them, and the
     rows that see them what the generic path makes of them (the queries off the vectors' alignment)."""
