@@ -1663,17 +1663,26 @@ kimkv_status launch_decode(const kimkv_storage* storage, const kimkv_decode_item
     } else {
         // Streamed K/V loads for long chunks (a workgroup streams at least
         // 2048 tokens), more than one round of resident workgroups (two
-        // per CU), or a launch that reads much: from about 96 MB of pages
-        // on, which no cache keeps until the next pass (48 lanes of up to
-        // 6000 tokens 37.8 -> 34.4 us, 16 of up to 4000 of 8 x 128 31.8 ->
-        // 28.4).  Cached loads for the short, latency-bound launches (20
+        // per CU), or a launch that surely reads 96 MB of pages: a lane of c
+        // chunks holds more than c - 1 full ones.  In a program other layers'
+        // pages and weights are read between two launches on the same pages,
+        // and then the streamed form is the faster one, with pages that lanes
+        // share too (launches on 6 batches in turn, and with 256 MB of reads
+        // between them, cached -> streamed: 48 lanes of up to 6000 tokens
+        // 36.9 -> 33.6 and 61.7 -> 36.2 us, 16 of up to 4000 of 8 x 128 39.6
+        // -> 36.0 and 65.4 -> 37.0, 32 lanes on 8 prefixes of 2048 26.8 ->
+        // 26.0 and 53.3 -> 27.5, on 8 of 8192 33.4 -> 37.2 and 60.3 -> 39.6,
+        // on one of 4096 20.0 -> 29.6 and 30.6 -> 32.2).  Repeated on one
+        // batch of 96 to 256 MB alone, which the last-level cache keeps, it
+        // is the slower one (30.2 -> 31.1 us for the 48 lanes).  Cached
+        // loads for the short, latency-bound launches (20
         // lanes of up to 900 tokens 10.2, streamed 11.1; 3 of up to 20000 of
-        // 8 x 64, 89 MB, 20.0 and 20.7), and where the engine launches:
-        // its lanes may share pages, which the caches serve (32 lanes on
-        // shared prefixes, 22 layers twice: 1165 us, streamed 1245).
+        // 8 x 64, 89 MB, 20.0 and 20.7), and where the engine launches: its
+        // lanes share prefixes and its layers' launches follow each other
+        // (32 lanes, 22 layers twice: 1165 us, streamed 1245).
         uint64_t const resident = 2ull * (storage->compute_units > 0 ? storage->compute_units : 256);
-        uint64_t const page_bytes =
-            4ull * total_chunks * chunk_tokens * storage->layout.kv_heads * storage->layout.head_dim;
+        uint64_t const page_bytes = 4ull * (total_chunks > lane_count ? total_chunks - lane_count : 0) * chunk_tokens
+            * storage->layout.kv_heads * storage->layout.head_dim;
         bool const stream_loads = chunk_tokens >= 2048 || static_cast<uint64_t>(grid.x) * grid.y > resident
             || (!records && writes == nullptr && page_bytes >= (96ull << 20));
         PoolView const pv = pool_view(*storage);
