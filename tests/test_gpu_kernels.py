@@ -258,8 +258,9 @@ def test_promotion_bit_exact(dev):
 
 # ---- decode ---------------------------------------------------------------------
 
-def _run_decode(dev, storage, lanes, query_heads, stream=None, chunk=None):
-    """lanes: list of (desc array, token_count, layer, query codes, scale); chunk forces the chunk length."""
+def _run_decode(dev, storage, lanes, query_heads, stream=None, chunk=None, q_off=0):
+    """lanes: list of (desc array, token_count, layer, query codes, scale); chunk forces the chunk length; the
+    queries lie q_off halves past a 16-byte boundary."""
     counts = [t for (_, t, _, _, _) in lanes]
     if chunk is None:
         chunk, prefix, total = storage.decode_plan(counts, query_heads)
@@ -271,11 +272,11 @@ def _run_decode(dev, storage, lanes, query_heads, stream=None, chunk=None):
     outs = []
     for i, (table, T, layer, q, scale) in enumerate(lanes):
         dbuf = dev.upload(table)
-        qbuf = dev.upload(q)
+        qbuf = dev.upload(np.concatenate([np.zeros(q_off, np.uint16), q]))
         obuf = dev.DeviceBuffer(query_heads * storage.head_dim * 2)
         wsz = dev.workspace_bytes(T, chunk, query_heads, storage.head_dim)
         wbuf = dev.DeviceBuffer(max(wsz, 4))
-        items[i] = (dbuf.ptr, len(table), T, layer, qbuf.ptr, wbuf.ptr if wsz else 0, obuf.ptr, scale)
+        items[i] = (dbuf.ptr, len(table), T, layer, qbuf.ptr + 2 * q_off, wbuf.ptr if wsz else 0, obuf.ptr, scale)
         keep += [dbuf, qbuf, wbuf]
         outs.append(obuf)
     ibuf = dev.upload(items)
@@ -286,7 +287,7 @@ def _run_decode(dev, storage, lanes, query_heads, stream=None, chunk=None):
 
 
 def _decode_case(dev, shape, token_counts, G, micro_tokens=8, extent_tokens=64, layer=None, seed=1,
-                 uniform_pages=None, chunk=None, repeat=1):
+                 uniform_pages=None, chunk=None, repeat=1, q_off=0):
     L, H, D = shape
     QH = H * G
     micro_cap = sum(t // micro_tokens + 2 for t in token_counts) + 8
@@ -311,7 +312,7 @@ def _decode_case(dev, shape, token_counts, G, micro_tokens=8, extent_tokens=64, 
     worst = 0.0
     first = None
     for _ in range(repeat):
-        outs, planned, total = _run_decode(dev, storage, lanes, QH, chunk=chunk)
+        outs, planned, total = _run_decode(dev, storage, lanes, QH, chunk=chunk, q_off=q_off)
         for got, want in zip(outs, wants):
             worst = max(worst, helpers.assert_attention_close(got, want))
         if first is None:
@@ -324,11 +325,12 @@ def _decode_case(dev, shape, token_counts, G, micro_tokens=8, extent_tokens=64, 
     return chunk, total
 
 
-def _write_then_decode(dev, fused, tables, T, news, lanes_meta, QH, chunk, shape, seed, cows):
+def _write_then_decode(dev, fused, tables, T, news, lanes_meta, QH, chunk, shape, seed, cows, off=0):
     """One storage populated from `tables`, each lane's new token at position T[i] (into its tail page, a
     fresh page, or a copy-on-write copy of a shared tail), then the decode of T[i] + 1 tokens: by
     kimkv_paged_decode_write_batch (fused) or kimkv_append_batch + kimkv_paged_decode_batch.  Returns the
-    outputs and every lane's gathered pages."""
+    outputs and every lane's gathered pages.  New rows and queries lie `off` halves past a 16-byte
+    boundary."""
     L, H, D = shape
     micro_cap = sum(t // 8 + 4 for t in T) + 16
     ext_cap = sum(t // 64 + 1 for t in T) + 2
@@ -339,14 +341,16 @@ def _write_then_decode(dev, fused, tables, T, news, lanes_meta, QH, chunk, shape
         keep.append(_populate(dev, storage, pools, table, _input(L, H, D, T[i], seed=seed * 100 + i)))
     jobs = np.zeros(len(T), dtype=dev.APPEND_JOB)
     ext_tables = []
-    src = dev.upload(news)            # [lane][2][H][D]
+    buf = dev.upload(np.concatenate([np.zeros(off, np.uint16), news.reshape(-1)]))   # [lane][2][H][D]
+    src = buf.ptr + 2 * off
+    keep.append(buf)
     for i, table in enumerate(tables):
         layer = lanes_meta[i]
         t = table.copy()
         tail = t[-1]
         j = jobs[i]
-        j["src_key"] = src.ptr + 2 * (i * 2) * H * D
-        j["src_value"] = src.ptr + 2 * (i * 2 + 1) * H * D
+        j["src_key"] = src + 2 * (i * 2) * H * D
+        j["src_value"] = src + 2 * (i * 2 + 1) * H * D
         j["layer_begin"], j["layer_count"], j["token_count"] = layer, 1, 1
         j["dst_kind"] = 0
         if tail["kind"] == 0 and tail["valid_tokens"] < 8 and i in cows:
@@ -375,11 +379,11 @@ def _write_then_decode(dev, fused, tables, T, news, lanes_meta, QH, chunk, shape
     items = np.zeros(len(lanes), dtype=dev.DECODE_ITEM)
     outs = []
     for i, (table, n, layer, q, scale) in enumerate(lanes):
-        dbuf, qbuf = dev.upload(table), dev.upload(q)
+        dbuf, qbuf = dev.upload(table), dev.upload(np.concatenate([np.zeros(off, np.uint16), q]))
         obuf = dev.DeviceBuffer(QH * D * 2)
         wsz = dev.workspace_bytes(n, chunk, QH, D)
         wbuf = dev.DeviceBuffer(max(wsz, 4))
-        items[i] = (dbuf.ptr, len(table), n, layer, qbuf.ptr, wbuf.ptr if wsz else 0, obuf.ptr, scale)
+        items[i] = (dbuf.ptr, len(table), n, layer, qbuf.ptr + 2 * off, wbuf.ptr if wsz else 0, obuf.ptr, scale)
         keep += [dbuf, qbuf, wbuf]
         outs.append(obuf)
     ibuf, pbuf, jbuf = dev.upload(items), dev.upload(prefix), dev.upload(jobs)
@@ -934,10 +938,12 @@ def test_decode_split_k_long_lanes(dev):
 
 
 def test_decode_combine_wide_heads_and_many_chunks(dev):
-    # Split-K merges with 2 and 4 dims per lane (D = 128, 256; generic path)
-    # and a lane of more than 64 chunks (the merge folds rounds of 64).
-    chunk, total = _decode_case(dev, (1, 2, 128), [300, 2600], G=4, seed=13)
-    assert total > 2
+    # Split-K merges with 2 and 4 dims per lane (D = 128: fast path; 96, 256:
+    # generic path) and a lane of more than 64 chunks (the merge folds rounds
+    # of 64).
+    for dim in (128, 96):
+        chunk, total = _decode_case(dev, (1, 2, dim), [300, 2600], G=4, seed=13)
+        assert total > 2
     chunk, total = _decode_case(dev, (1, 1, 256), [700, 2000], G=2, seed=14)
     assert total > 2
     chunk, total = _decode_case(dev, (1, 4, 64), [20000, 33], G=8, seed=15)
@@ -997,9 +1003,9 @@ def test_decode_guided_slices(dev):
     # Persistent workgroups taking (slice, lane, kv head) units from the
     # device counter: ragged lanes with one to six slices (one-slice lanes
     # written directly, empty slices from 64-alignment), the longest slices
-    # the table holds (T/2 <= 65536), group sizes 16 and 1, generic head dims
-    # and unaligned pages (generic wave path), and many launches in a row
-    # (counter slots reused after their reset).
+    # the table holds (T/2 <= 65536), group sizes 16 and 1, head dim 128,
+    # unaligned pages (generic path), and many launches in a row (counter
+    # slots reused after their reset).
     GU = dev.DECODE_GUIDED | 64
     _decode_case(dev, (2, 4, 64), [1, 5, 66, 100, 131, 396, 397, 4000, 12345, 33000], G=8, seed=60, chunk=GU)
     _decode_case(dev, (1, 4, 64), [130000, 70000, 64, 8193], G=8, seed=61, chunk=GU)
@@ -1040,7 +1046,7 @@ def test_decode_head_split(dev):
     _decode_case(dev, (1, 4, 64), [32769, 10944, 5, 70000], G=8, seed=21, chunk=32832 | S)
     _decode_case(dev, (2, 2, 64), [130, 700, 3000], G=16, seed=22, chunk=512 | S)
     _decode_case(dev, (2, 8, 64), [70, 333, 4100], G=1, seed=23, chunk=4096 | S)
-    # A table that is not 8-aligned takes the generic path in the first wave.
+    # A table that is not 8-aligned takes the generic path, a quarter of the chunk in each wave.
     _decode_case(dev, (2, 4, 64), [17, 200, 3000], G=8, micro_tokens=6, extent_tokens=48, seed=24,
                  uniform_pages=True, chunk=1024 | S)
 
@@ -1070,9 +1076,35 @@ def test_decode_head_dim_128_guided(dev):
     _decode_case(dev, (2, 4, 128), [1, 63, 300, 1000, 5000], G=4, seed=82, chunk=dev.DECODE_GUIDED | 64)
 
 
+@pytest.mark.parametrize("mode", ["four_heads", "head_split", "guided"])
+def test_decode_head_dim_128_unaligned_queries(dev, mode):
+    """Queries two bytes past the vectors' alignment."""
+    chunk = {"four_heads": 256, "head_split": 256 | dev.DECODE_HEAD_SPLIT, "guided": dev.DECODE_GUIDED | 64}[mode]
+    _decode_case(dev, (2, 4, 128), [1, 31, 64, 100, 300, 1000], G=4, seed=99, chunk=chunk, q_off=1)
+
+
+def test_decode_and_prefill_head_dim_128_all_scores_infinite(dev):
+    """Keys whose scores are all -inf leave a denominator of 0 and an output of 0, not NaN."""
+    H, D, G, T, n = 1, 128, 4, 70, 40
+    storage = dev.Storage(1, H, D, 32, 4)
+    pools = oracle.HostPools(1, H, D, 32, 4)
+    table = helpers.hetero_table(T, helpers.SlotAllocator(32, 4, seed=3))
+    inp = _input(1, H, D, T, seed=100)
+    inp[0, 0, :, :, 0] = 0xFC00   # -inf
+    _populate(dev, storage, pools, table, inp)
+    q = np.zeros((n, G, D), np.uint16)
+    q[:, :, 0] = 0x3C00           # 1
+    assert np.all(_prefill_rows(dev, storage, table, T, n, H * G, q) & 0x7FFF == 0)
+    for chunk in (128, 128 | dev.DECODE_HEAD_SPLIT):
+        outs, _, _ = _run_decode(dev, storage, [(table, T, 0, q[0].reshape(-1), 1.0)], H * G, chunk=chunk)
+        assert np.all(outs[0] & 0x7FFF == 0)
+
+
+@pytest.mark.parametrize("off", [0, 1])
 @pytest.mark.parametrize("mode", ["four_heads", "head_split"])
-def test_decode_head_dim_128_writes(dev, mode):
-    """The 128-dim fast path's fused token write: outputs and pages as append-then-decode gives them."""
+def test_decode_head_dim_128_writes(dev, mode, off):
+    """The 128-dim fast path's fused token write: outputs and pages as append-then-decode gives them, with
+    new rows and queries on the vectors' alignment and two bytes past it."""
     shape, G = (2, 4, 128), 4
     L, H, D = shape
     T = [5, 8, 31, 32, 63, 64, 100, 700, 1303]
@@ -1082,8 +1114,8 @@ def test_decode_head_dim_128_writes(dev, mode):
     news = oracle.synth_rows(len(T) * 2 * H * D, 84, 0, D).reshape(len(T), 2, H, D)
     layers = [i % L for i in range(len(T))]
     chunk = {"four_heads": 256, "head_split": 256 | dev.DECODE_HEAD_SPLIT}[mode]
-    a, pa, total = _write_then_decode(dev, False, tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8})
-    b, pb, _ = _write_then_decode(dev, "slots_prefix", tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8})
+    a, pa, total = _write_then_decode(dev, False, tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8}, off)
+    b, pb, _ = _write_then_decode(dev, "slots_prefix", tables, T, news, layers, H * G, chunk, shape, 85, {0, 6, 8}, off)
     assert total > len(T)
     for i in range(len(T)):
         assert np.array_equal(pa[i], pb[i]) and np.array_equal(a[i], b[i]), (mode, i)
