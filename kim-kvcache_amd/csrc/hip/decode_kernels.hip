@@ -59,9 +59,10 @@ constexpr bool fast_head_dim(uint32_t dim) { return dim == 64 || dim == 128; }
 // A K or V^T operand load: non-temporal (streamed past the caches) for long
 // chunks and large launches, where every byte is read once and the
 // streaming hint keeps HBM busier (7.1 vs 6.2 TB/s in a read probe; the
-// 128-lane x 32k launch is 0.656 instead of 0.640 ms without it); cached for
-// short chunks in small, latency-bound launches (the 32-lane shared-prefix
-// layer: 24.9 instead of 26.4 us).
+// 128-lane x 32k launch is 0.656 instead of 0.640 ms without it), and for
+// item launches of 96 MB and more, whose pages no cache holds by the time
+// they are read again; cached for short chunks in small, latency-bound
+// launches (the 32-lane shared-prefix layer: 24.9 instead of 26.4 us).
 template <bool kStream>
 __device__ __attribute__((always_inline)) inline half8_t load_kv(const uint16_t* p)
 {
@@ -110,8 +111,10 @@ __device__ inline half8_t load_row8(const uint16_t* p)
 // by the MFMAs.  kDim = 128 keeps the registers of kDim = 64 by taking 32
 // tokens a step: a step is 16 KiB of K/V per wave either way, two steps in
 // flight.  16 lanes of 500..4000 tokens, 8 kv heads x 128, 4 query heads each
-// (137 MB): 42.5 us with the merge, 1205 us on the generic path, which reads
-// K and V once per query head in 2-byte loads.
+// (137 MB): 38.0 us with the merge, 1208 us on the generic path, which reads
+// K and V once per query head in 2-byte loads.  Errors against 64 bits are
+// those of rounding the results to fp16 alone on both paths (2.05e-4, queries
+// of 1, 4 and 12 times unit variance, lanes of up to 9000 tokens).
 template <uint32_t kDim, bool kStream>
 __device__ WavePartial<kDim> decode_wave_fast(const GroupEntry* groups, const GroupResolver& res,
                                               const kimkv_decode_item& item, uint32_t h, uint32_t G, uint32_t g0,
@@ -1396,7 +1399,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 // unrolled rows run once, so their instructions come from memory, and 64 of
 // them cost more than the second round of loads that 17 rows take (200 lanes
 // of 100..900 tokens with the decode 41.0 -> 32.5 us, 8 lanes of up to 3000
-// 12.6 -> 10.6, 48 lanes of up to 6000 39.2 -> 37.8).
+// 12.6 -> 10.6, 48 lanes of up to 6000 39.2 -> 37.8).  The host knows the
+// lanes' mean, not the longest: one lane of 118 chunks among 15 or 47 of one
+// costs 0.8 us more by 16 rows (19.1 -> 19.9).  Both in one kernel, chosen by
+// the lane, serve that launch (18.4) and cost the others what 16 rows gain
+// (31.1 -> 32.9, 11.4 -> 12.5); rows staged in LDS by a loop of direct loads
+// are no faster than either.
 constexpr unsigned kCombineHeads = 4;
 
 // Where the merge of a record launch finds its lanes: each lane's output

@@ -398,7 +398,8 @@ bool linear_fits(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* 
 void linear_launch(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t* w, uint32_t out, void* y, bool f32,
                    float beta, hipStream_t stream)
 {
-    // One workgroup per CU: as many feature tiles each as that takes, up to
+    // One workgroup per CU up to 16384 features (32000 make 500): as many
+    // feature tiles each as that takes, up to
     // four, or the rows in two blocks where that still fits (the second
     // block, on the same XCD when the tiles are a multiple of 8, reads the
     // weights from its L2: 5632 x 2048, 32 rows, 11.7 us as one, 8.6 as two).

@@ -26,7 +26,7 @@
 // registers) and hands its softmax weights to the matrix cores in two fp16
 // parts, so that they keep the precision of fp32 weights (two ragged chunks
 // of up to 256 tokens on contexts of up to 1500, 8 kv heads x 128, 4 query
-// heads each: 35.8 us, 4440 us on the generic path).
+// heads each: 35.9 us, 4449 us on the generic path a row at a time).
 // Tables that do not keep 8-token groups aligned, head dims other than 64 and
 // 128 and group sizes that do not divide 16 take a generic path, eight rows at
 // a time.
@@ -58,7 +58,10 @@ struct PrefillDims {
     static constexpr uint32_t kDb = kDim / 16;           // 16-dim blocks of O
     // Softmax weights as two fp16 parts, p = hi + lo (~22 bits, where the
     // generic path these shapes took before holds fp32 weights); the weights
-    // are then shifted up so that lo stays a normal number for small ones.
+    // are then shifted up so that lo is a normal number down to 2^-9 of the
+    // largest weight, and the parts hold any to 2^-32 of it.  Errors against
+    // 64 bits are those of rounding the results to fp16 alone on both paths
+    // (2.07e-4, queries of 1, 4 and 12 times unit variance).
     static constexpr bool kSplitP = kDim == 128;
     static constexpr float kWeightShift = kSplitP ? 7.0f : 0.0f;
 };
