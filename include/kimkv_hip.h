@@ -603,19 +603,20 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
  * y = the residual stream fuses the residual add.  Few rows (16; 32 up to
  * 12288 features, 64 up to 4096 features of sums up to 4096 and 16 MB of
  * weights; in a multiple of 64, x and weight 16-byte aligned) run on this
- * library's own kernel, the rest on hipBLASLt's first heuristic choice, kept per exact problem (rows,
- * in, out, output type, beta != 0) and stream.  Which of the two a call takes
- * follows from the call alone, not from earlier calls, unless
- * kimkv_linear_tune chose for its problem: then the tuned algorithm, or the
- * library's best where the own kernel won and the addresses are not aligned. */
+ * library's own kernel, the rest on hipBLASLt's first heuristic choice, kept
+ * per exact problem (rows, in, out, output type, beta != 0) and stream.
+ * Which of the two a call takes follows from the call alone, not from earlier
+ * calls, unless kimkv_linear_tune chose for its problem: then the tuned
+ * algorithm, or the library's best where the own kernel won and the addresses
+ * are not aligned. */
 kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features, const uint16_t* weight,
                           uint32_t out_features, void* y, int y_f32, float beta, kimkv_stream_t stream);
 /* Times hipBLASLt's leading candidates and, where it fits, this library's own
- * kernel for this exact problem by the GPU's work alone (the stream
- * is synchronized; y is overwritten or accumulated into several times, so
- * pass scratch contents) and makes the first of those within 2% of the
- * fastest the one kimkv_linear uses for the problem on this stream, so that
- * one process chooses as the next does.  Successive timed products cycle through the
+ * kernel for this exact problem by the GPU's work alone (the stream is
+ * synchronized; y is overwritten or accumulated into several times, so pass
+ * scratch contents) and makes the first of those within 2% of the fastest the
+ * one kimkv_linear uses for the problem on this stream, so that one process
+ * chooses as the next does.  Successive timed products cycle through the
  * weight_count weight matrices (e.g. every layer's), so the weights are read
  * from HBM as in a forward pass, not from a warm cache.  No counterpart in
  * the reference (cuBLAS picks its own algorithm). */

@@ -399,8 +399,8 @@ void linear_launch(const uint16_t* x, uint32_t rows, uint32_t in, const uint16_t
                    float beta, hipStream_t stream)
 {
     // One workgroup per CU up to 16384 features (32000 make 500): as many
-    // feature tiles each as that takes, up to
-    // four, or the rows in two blocks where that still fits (the second
+    // feature tiles each as that takes, up to four, or the rows in two blocks
+    // where that still fits (the second
     // block, on the same XCD when the tiles are a multiple of 8, reads the
     // weights from its L2: 5632 x 2048, 32 rows, 11.7 us as one, 8.6 as two).
     uint32_t const tiles = (out + 15) / 16;
