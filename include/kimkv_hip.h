@@ -611,15 +611,16 @@ kimkv_status kimkv_decode_timing_busy(double* busy_ms);
  * are not aligned. */
 kimkv_status kimkv_linear(const uint16_t* x, uint32_t rows, uint32_t in_features, const uint16_t* weight,
                           uint32_t out_features, void* y, int y_f32, float beta, kimkv_stream_t stream);
-/* Times hipBLASLt's leading candidates and, where it fits, this library's own
- * kernel for this exact problem by the GPU's work alone (the stream is
- * synchronized; y is overwritten or accumulated into several times, so pass
- * scratch contents) and makes the first of those within 2% of the fastest the
- * one kimkv_linear uses for the problem on this stream, so that one process
- * chooses as the next does.  Successive timed products cycle through the
- * weight_count weight matrices (e.g. every layer's), so the weights are read
- * from HBM as in a forward pass, not from a warm cache.  No counterpart in
- * the reference (cuBLAS picks its own algorithm). */
+/* Times hipBLASLt's leading candidates for this exact problem by the GPU's
+ * work alone and takes the first of those within 2% of the fastest, so that
+ * one process chooses as the next does; where this library's own kernel fits,
+ * times the two call after call.  The stream is synchronized, and y is
+ * overwritten or accumulated into several times, so pass scratch contents.
+ * The winner is the one kimkv_linear uses for the problem on this stream.
+ * Successive timed products cycle through the weight_count weight matrices
+ * (e.g. every layer's), so the weights are read from HBM as in a forward
+ * pass, not from a warm cache.  No counterpart in the reference (cuBLAS picks
+ * its own algorithm). */
 kimkv_status kimkv_linear_tune(const uint16_t* x, uint32_t rows, uint32_t in_features,
                                const uint16_t* const* weights, uint32_t weight_count, uint32_t out_features, void* y,
                                int y_f32, float beta, kimkv_stream_t stream);

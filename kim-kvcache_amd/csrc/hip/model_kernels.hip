@@ -684,8 +684,8 @@ kimkv_status kimkv_linear_tune(const uint16_t* x, uint32_t rows, uint32_t in_fea
     constexpr int kCandidates = 16;
     constexpr int kRounds = 3;   // a contender's time is its best round: one-off interference does not decide
     constexpr int kReps = 6;
-    // Two candidates this near are one: the first of them is taken.  Best
-    // rounds of one candidate differ by up to 1.5% between processes.
+    // Of candidates this near each other the first is taken: the best rounds
+    // of one differ by up to 1.5% between processes.
     constexpr float kTie = 1.02f;
     if (weights == nullptr || weight_count == 0) return KIMKV_INVALID_ARGUMENT;
     for (uint32_t i = 0; i < weight_count; ++i) {
@@ -708,82 +708,98 @@ kimkv_status kimkv_linear_tune(const uint16_t* x, uint32_t rows, uint32_t in_fea
         lt_destroy(p);
         return n < 1 ? KIMKV_SUBMISSION_FAILED : KIMKV_RUNTIME_UNAVAILABLE;
     }
-    float time_ms[kCandidates + 1];
+    float time_ms[kCandidates];
     bool usable[kCandidates + 1];
     for (int a = 0; a < n; ++a) {
-        time_ms[a] = 0.0f;
         usable[a] = lt_run(st, *ctx, p, cand[a].algo, x, weights[0], y, beta, s) == HIPBLAS_STATUS_SUCCESS;
     }
     // The kernel of few rows is one more candidate, n.
     bool own = true;
     for (uint32_t i = 0; i < weight_count; ++i) own = own && linear_fits(x, rows, in_features, weights[i], out_features);
     usable[n] = own;
-    time_ms[n] = 0.0f;
     if (own) {
         linear_launch(x, rows, in_features, weights[0], out_features, y, y_f32 != 0, beta, s);
         usable[n] = launch_status() == KIMKV_OK;
     }
-    auto product = [&](int a, const uint16_t* w) {
-        if (a != n) return lt_run(st, *ctx, p, cand[a].algo, x, w, y, beta, s) == HIPBLAS_STATUS_SUCCESS;
-        linear_launch(x, rows, in_features, w, out_features, y, y_f32 != 0, beta, s);
-        return launch_status() == KIMKV_OK;
-    };
-    // Round 0 finds the contenders.  In the rounds that decide, the products
-    // are queued behind a wait, so that the events bracket the GPU's work
-    // alone: a call of the library's takes 10 us of host work, as long as a
-    // product of 128 rows, and times of that decided between candidates 5%
-    // apart one way in one process and the other way in the next.  A wait too
-    // short for the host is doubled, for this and the candidates after it.
-    float limit = INFINITY;
-    uint32_t ticks = 8000;
-    constexpr uint32_t kMostTicks = 64000;
-    for (int round = 0; round <= kRounds; ++round) {
-        for (int a = 0; a <= n; ++a) {
-            if (!usable[a] || time_ms[a] > limit) continue;
-            float ms = 0.0f;
-            bool ok = true;
-            for (bool late = true; late && ok;) {
-                if (round != 0) wait_kernel<<<1, 64, 0, s>>>(ticks);
-                ok = hipEventRecord(e0, s) == hipSuccess;
-                for (int i = 0; i < kReps && ok; ++i) {
-                    ok = product(a, weights[(static_cast<uint32_t>(round * kReps + i) + static_cast<uint32_t>(a)) % weight_count]);
+    // Time per product of `reps` of candidate a, or INFINITY on an error.  The
+    // matrices are taken in turn over all timings, so each was last read
+    // weight_count products ago, whoever read it.  wait: the products are
+    // queued behind a wait, so that the events bracket the GPU's work alone;
+    // one too short for the host is doubled, for this and the candidates
+    // after it, and the products are timed again (a busy host may need the
+    // longest several times).
+    uint32_t ticks = 1300;   // a product queued
+    constexpr uint32_t kMostTicks = 10000;
+    constexpr int kAttempts = 8;
+    uint32_t turn = 0;
+    auto timed = [&](int a, int reps, bool wait) {
+        float ms = 0.0f;
+        bool ok = true;
+        bool late = true;
+        for (int attempt = 0; attempt < kAttempts && late && ok; ++attempt) {
+            if (wait) wait_kernel<<<1, 64, 0, s>>>(ticks * static_cast<uint32_t>(reps));
+            ok = hipEventRecord(e0, s) == hipSuccess;
+            for (int i = 0; i < reps && ok; ++i) {
+                const uint16_t* w = weights[turn++ % weight_count];
+                if (a == n) {
+                    linear_launch(x, rows, in_features, w, out_features, y, y_f32 != 0, beta, s);
+                    ok = launch_status() == KIMKV_OK;
+                } else {
+                    ok = lt_run(st, *ctx, p, cand[a].algo, x, w, y, beta, s) == HIPBLAS_STATUS_SUCCESS;
                 }
-                hipError_t const begun = hipEventQuery(e0);
-                if (begun == hipErrorNotReady) static_cast<void>(hipGetLastError());   // the answer hoped for, no error
-                late = round != 0 && ticks < kMostTicks && begun == hipSuccess;
-                if (late) ticks *= 2;
-                ok = ok && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess
-                    && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
             }
-            if (!ok) {
-                usable[a] = false;
-            } else if (round <= 1 || ms < time_ms[a]) {
-                time_ms[a] = ms;
-            }
+            hipError_t const begun = hipEventQuery(e0);
+            if (begun == hipErrorNotReady) static_cast<void>(hipGetLastError());   // the answer hoped for, no error
+            late = wait && begun == hipSuccess;
+            if (late && ticks < kMostTicks) ticks *= 2;
+            ok = ok && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess
+                && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
         }
-        if (round == 0) {
-            for (int a = 0; a < n; ++a) {   // of the library's: its best is wanted even where the own kernel wins
-                if (usable[a]) limit = std::min(limit, 1.25f * time_ms[a]);
-            }
-            for (int a = 0; a <= n; ++a) {
-                if (time_ms[a] > limit) time_ms[a] = INFINITY;
-            }
+        return ok ? ms / static_cast<float>(reps) : INFINITY;
+    };
+    // Of the library's candidates, by the GPU's work: a call of the library's
+    // takes 10 us of host work, as long as a product of 128 rows, and times
+    // of that decided between candidates 5% apart one way in one process and
+    // the other way in the next.  A short round finds the contenders, after
+    // each candidate's code and every matrix's translations have been loaded.
+    float limit = INFINITY;
+    for (int a = 0; a < n; ++a) {
+        for (uint32_t i = 0; usable[a] && i < 1 + weight_count / static_cast<uint32_t>(n); ++i) {
+            usable[a] = lt_run(st, *ctx, p, cand[a].algo, x, weights[turn++ % weight_count], y, beta, s) == HIPBLAS_STATUS_SUCCESS;
         }
     }
-    // The earliest candidate that ties with the fastest, of all and (for
-    // calls the own kernel does not take) of the library's.
-    auto choose = [&](int count) {
-        float least = INFINITY;
-        for (int a = 0; a < count; ++a) {
-            if (usable[a]) least = std::min(least, time_ms[a]);
+    for (int a = 0; a < n; ++a) {
+        time_ms[a] = usable[a] ? timed(a, 2, true) : INFINITY;
+        limit = std::min(limit, 1.25f * time_ms[a]);
+    }
+    for (int a = 0; a < n; ++a) {
+        usable[a] = usable[a] && time_ms[a] <= limit;
+        time_ms[a] = INFINITY;
+    }
+    float least = INFINITY;
+    for (int round = 0; round < kRounds; ++round) {
+        for (int a = 0; a < n; ++a) {
+            if (usable[a]) time_ms[a] = std::min(time_ms[a], timed(a, kReps, true));
+            least = std::min(least, time_ms[a]);
         }
-        for (int a = 0; a < count; ++a) {
-            if (usable[a] && time_ms[a] <= least * kTie) return a;
+    }
+    int library = -1;
+    for (int a = 0; a < n && library < 0; ++a) {
+        if (time_ms[a] < INFINITY && time_ms[a] <= least * kTie) library = a;
+    }
+    // Between that and the own kernel, call after call: the host's part,
+    // which a program of such short products waits for, differs (20 rows,
+    // 2048 x 11264: 11.1 us of GPU time against 10.4, but 11.1 against 11.6
+    // a call).
+    int best = library;
+    if (usable[n] && library >= 0) {
+        float call[2] = {INFINITY, INFINITY};
+        for (int round = 0; round < kRounds; ++round) {
+            call[0] = std::min(call[0], timed(library, kReps, false));
+            call[1] = std::min(call[1], timed(n, kReps, false));
         }
-        return -1;
-    };
-    int const best = choose(n + 1);
-    int const library = choose(n);
+        if (call[1] <= call[0]) best = n;
+    }
     static_cast<void>(hipEventDestroy(e0));
     static_cast<void>(hipEventDestroy(e1));
     if (library < 0) {

@@ -257,6 +257,26 @@ def test_linear_rows_by_length_of_sum(dev, rows, fin, own):
     assert np.array_equal(got[0], got[1]) != own
 
 
+def test_linear_tune_keeps_the_own_kernel(dev):
+    """A product of few rows whose library call costs 1.3 times the own kernel's and more: tuned, it has the
+    bits of the untuned one, the own kernel's."""
+    rows, fin, fout, layers = 20, 2048, 2048, 8
+    x = _f16(np.random.default_rng(10), (rows, fin), 1.0)
+    xb, wb = dev.upload(x.view(np.uint16)), dev.DeviceBuffer(2 * layers * fin * fout)
+    dev.fill_rows(wb.ptr, layers * fin * fout, 7, 0, fin)
+    dev.sync()
+    got = []
+    for tuned in (False, True):
+        stream, yb = dev.Stream(), dev.DeviceBuffer(rows * fout * 4)
+        if tuned:
+            dev.linear_tune(xb.ptr, rows, fin, [wb.ptr + 2 * i * fin * fout for i in range(layers)], fout, yb.ptr, True,
+                            0.0, stream)
+        dev.linear(xb.ptr, rows, fin, wb.ptr, fout, yb.ptr, True, 0.0, stream)
+        dev.sync(stream)
+        got.append(dev.download(yb.ptr, (rows, fout), np.float32))
+    assert np.array_equal(got[0], got[1])
+
+
 def test_linear_tune_chooses_alike(dev):
     """A problem whose candidates lie a few percent apart, its weights read
     from HBM (24 layers' matrices), on a host that is busy otherwise: every
