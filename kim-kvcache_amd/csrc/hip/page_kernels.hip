@@ -201,6 +201,10 @@ __device__ inline void copy_tokens_wide(const AppendDivisors& dv, uint32_t n, co
     }
 }
 
+// kHuge: the layout has offsets past 32 bits (append_huge), so every copy goes
+// element by element at 64-bit offsets.  An instance of its own, as the two
+// forms of offsets in one kernel cost the 64-lane append 0.15 us of 15.8.
+template <bool kHuge>
 __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_append_job* jobs,
                                                         uint32_t job_count, AppendDivisors dv)
 {
@@ -220,15 +224,20 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
     }
     uint32_t const tid = threadIdx.x;
 
+    auto k_el = [](uint32_t cap, uint32_t dim, uint32_t t, uint32_t d) -> uint64_t {
+        return kHuge ? k_offset(cap, dim, t, d) : k_at(cap, dim, t, d);
+    };
+    auto v_el = [](uint32_t cap, uint32_t dim, uint32_t t, uint32_t d) -> uint64_t {
+        return kHuge ? v_offset(cap, dim, t, d) : v_at(cap, dim, t, d);
+    };
+
     // The copied positions lie below the written ones: neither waits for the other.
     if (job.cow_tokens != 0) {
         uint32_t const scap = pool_tokens(P, job.cow_kind);
         uint16_t const* src = page_base(P, job.cow_kind, job.cow_slot, scap);
         uint32_t const n = job.cow_tokens;
         if (src != nullptr && n <= scap && n <= dcap && n <= job.dst_token) {
-            // The copy's offsets from the layer's blocks are 32 bits (64: the 64-lane append 0.2 us slower).
-            bool const small = ((P.micro_slot_elements | P.extent_slot_elements) >> 32) == 0;
-            if (small && ((D | scap | dcap) & 7u) == 0) {
+            if (!kHuge && ((D | scap | dcap) & 7u) == 0) {
                 copy_tokens_wide(dv, n, src + head_block(P, scap, layer, 0), scap, dst + head_block(P, dcap, layer, 0), dcap);
             } else {
                 uint32_t const per_head = n * D;
@@ -239,8 +248,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
                     uint32_t const d = rem - t * D;
                     uint64_t const sh = head_block(P, scap, layer, h);
                     uint64_t const dh = head_block(P, dcap, layer, h);
-                    dst[dh + k_offset(dcap, D, t, d)] = src[sh + k_offset(scap, D, t, d)];
-                    dst[dh + v_offset(dcap, D, t, d)] = src[sh + v_offset(scap, D, t, d)];
+                    dst[dh + k_el(dcap, D, t, d)] = src[sh + k_el(scap, D, t, d)];
+                    dst[dh + v_el(dcap, D, t, d)] = src[sh + v_el(scap, D, t, d)];
                 }
             }
         }
@@ -252,7 +261,7 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
     const uint16_t* sk = job.src_key + layer_off;
     const uint16_t* sv = job.src_value + layer_off;
     uint32_t const stride = job.src_token_stride;
-    bool const src_aligned = wide_dim(D) && (stride & 7u) == 0
+    bool const src_aligned = !kHuge && (D & 7u) == 0 && (stride & 7u) == 0
         && ((reinterpret_cast<uintptr_t>(sk) | reinterpret_cast<uintptr_t>(sv)) & 15u) == 0;
     if (src_aligned) {
         // K: 16-byte pieces of 8 dims of one token (contiguous in source and page).
@@ -303,8 +312,8 @@ __global__ __launch_bounds__(kBlock) void append_kernel(PoolView P, const kimkv_
         uint64_t const so = layer_off + static_cast<uint64_t>(t) * job.src_token_stride + rem;
         uint64_t const dh = head_block(P, dcap, layer, h);
         uint32_t const pt = job.dst_token + t;
-        dst[dh + k_offset(dcap, D, pt, d)] = job.src_key[so];
-        dst[dh + v_offset(dcap, D, pt, d)] = job.src_value[so];
+        dst[dh + k_el(dcap, D, pt, d)] = job.src_key[so];
+        dst[dh + v_el(dcap, D, pt, d)] = job.src_value[so];
     }
 }
 
@@ -662,6 +671,13 @@ __global__ __launch_bounds__(kBlock) void fill_kv_kernel(uint16_t* out, uint32_t
 using namespace kimkv;
 
 namespace {
+// Whether a layer's block of some page (from which the copied tails' offsets
+// count) or a head's (k_at, v_at) holds more elements than 32 bits count.
+bool append_huge(const PoolView& p)
+{
+    return ((p.micro_slot_elements | p.extent_slot_elements) >> 32) != 0 || p.dim > kMaxDim32;
+}
+
 AppendDivisors append_divisors(const kimkv_storage& s)
 {
     uint32_t const D = s.layout.head_dim;
@@ -681,8 +697,12 @@ kimkv_status kimkv_append_batch(const kimkv_storage* storage, const kimkv_append
     dim3 const grid(job_count, max_layer_count);
     void* start = nullptr;
     kernel_timing_begin(TimedKernel::Append, native(stream), &start);
-    append_kernel<<<grid, kBlock, 0, native(stream)>>>(pool_view(*storage), device_jobs, job_count,
-                                                         append_divisors(*storage));
+    PoolView const pv = pool_view(*storage);
+    if (append_huge(pv)) {
+        append_kernel<true><<<grid, kBlock, 0, native(stream)>>>(pv, device_jobs, job_count, append_divisors(*storage));
+    } else {
+        append_kernel<false><<<grid, kBlock, 0, native(stream)>>>(pv, device_jobs, job_count, append_divisors(*storage));
+    }
     kimkv_status const status = launch_status();
     kernel_timing_end(TimedKernel::Append, native(stream), start);
     return status;
